@@ -1,14 +1,32 @@
 // Device-side building blocks of the Born propagator on CDNA4 (gfx950).
 //
 // march_kernel advances one or two pressure fields by one leapfrog step of
-// the 8th-order constant-density acoustic operator.  A block of WY 64-lane
-// wavefronts owns a 64 x (RY*WY) cell tile of the xy plane (one wavefront per
-// x row group, RY rows per thread) and a chunk of z planes.  z neighbours
-// live in a 9-deep register queue per row; x/y neighbours of the current
-// plane come from an LDS tile with a 4-cell halo.  The loop is software
-// pipelined: the loads of plane z+1 (the queue's new leading plane, the LDS
-// halo and the op's pointwise inputs) are issued before plane z is computed,
-// so HBM latency overlaps the stencil arithmetic.
+// the 8th-order constant-density acoustic operator.  A block owns a tile of
+// the xy plane and a chunk of z planes, which it marches.  z neighbours live
+// in a 9-deep register queue per cell; x/y neighbours of the current plane
+// come from an LDS tile with a 4-cell halo.  The loop is software pipelined:
+// the loads of plane z+1 (the queue's new leading plane, the LDS halo and the
+// op's pointwise inputs) are issued before plane z is computed.
+//
+// What bounds it (MI355X, FP32).  At 304^3 memory: with the arithmetic and the
+// LDS exchange left out a launch takes as long.  At 160^3 (fields that fit
+// the 256 MB memory-side cache) a plane's loads and its arithmetic take about
+// as long as each other, and the 8 planes that a chunk shares with its
+// neighbours weigh.  At 64^3 latency: the launch, the chunk's first loads and
+// the planes marched one after the other.
+//   - A plane needs one barrier, not two: the LDS tile is double, and the halo
+//     loaded kH planes ahead waits in the loading thread's own LDS place.
+//   - Addresses are a scalar base that moves by a plane plus a lane offset
+//     that does not change: no address arithmetic per load and plane.
+//   - Chunks are marched up and down in turn, and turned round from one step
+//     to the next (Grid::back): neighbours read the planes they share
+//     together, and a step starts with the planes the last one ended with.
+//   - Four cells per lane (16-byte loads) where nx allows; the smallest tiles
+//     are one wavefront, whose barrier waits for nobody.
+// Together, fastest shape, us per step: 304^3 adjoint state 142.8 -> 130.9,
+// reference adjoint 233 -> 200, source propagation 79.9 -> 72.0, 24-bit
+// forward 194 -> 158; 160^3 forward 32.6 -> 30.0, adjoint state 24.9 -> 21.1,
+// source propagation 15.7 -> 12.6.
 //
 // What the step does with the Laplacian is supplied by an immutable "op"
 // functor inlined into the kernel: sponge, source injection, Born scatter,
@@ -38,6 +56,7 @@ struct Grid {
   int ntx, nty, ntz;  // tiles along x, y and z chunks
   int zc;             // planes per z chunk
   uint32_t plane;     // nx*ny
+  int back;           // 1: every z chunk is marched the other way
 };
 
 // Per-axis sponge factors: bound[min(edge_x, edge_y, edge_z)] equals
@@ -54,14 +73,33 @@ struct Points {
 
 // Receivers: every receiver plane z has a slot; rmap[slot][y][x] is the first
 // receiver at that cell (or -1), rnext[] chains receivers sharing a cell.
+//
+// A step touches one value per receiver cell, indexed by the cell's first
+// receiver: the forward leaves the new r there (the receivers' samples of a
+// window of steps are added to the traces afterwards, rec_accum_kernel), the
+// adjoints take from there what is injected (computed for a window of steps
+// beforehand, rec_inject_kernel).  Reading and writing the eight trace
+// samples of a receiver inside the step was a chain of three dependent loads
+// and a store per cell of a lane that the whole launch waited for.
 struct RecMap {
   const int *plane_slot;  // [nz], -1 when the plane has no receiver
   const int *rmap;        // [nslots][ny][nx]
   const int *rnext;       // [nrec]
   int nrec;
   int ntb;                // trace length (nt_big)
+  int shared;             // some cell holds more than one receiver
 };
 
+// The address `b` bytes (uniform, a scalar addition) past p, and the T at byte
+// offset o (a lane's, 32 bits) from a base: one load with a scalar base and
+// a vector offset.
+__device__ __forceinline__ const char *adv(const void *p, uint64_t b) {
+  return (const char *)p + b;
+}
+template <class T>
+__device__ __forceinline__ const T &ldb(const char *p, uint32_t o) {
+  return *(const T *)(p + (uint64_t)o);
+}
 // element at 32-bit element offset o (fields are < 2^30 cells)
 template <class T>
 __device__ __forceinline__ T &at(T *p, uint32_t o) {
@@ -126,27 +164,50 @@ __device__ __forceinline__ void st_b64(void *p, uint32_t off, uint64_t v) {
                  : : "v"(off), "v"(v), "s"(p) : "memory");
 }
 
+// A store of more than 8 bytes reads its data registers over more than one
+// cycle: one wait state before they may be written again.
+template <bool NT>
+__device__ __forceinline__ void st_b128(void *p, uint32_t off, uint4 v) {
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  const u4 w = {v.x, v.y, v.z, v.w};
+  if constexpr (NT)
+    asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 nt\n\ts_nop 1"
+                 : : "v"(off), "v"(w), "s"(p) : "memory");
+  else
+    asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2\n\ts_nop 1"
+                 : : "v"(off), "v"(w), "s"(p) : "memory");
+}
+
+// VX consecutive floats in LDS (VX = 2, 4: aligned to all of them)
+template <int VX>
+__device__ __forceinline__ void ld_lds(const float *p, float (&v)[VX]) {
+  if constexpr (VX == 1) {
+    v[0] = p[0];
+  } else {
+    typedef float vec __attribute__((ext_vector_type(VX)));
+    const vec w = *(const vec *)p;
+#pragma unroll
+    for (int i = 0; i < VX; i++) v[i] = w[i];
+  }
+}
+template <int VX>
+__device__ __forceinline__ void st_lds(float *p, const float (&v)[VX]) {
+  if constexpr (VX == 1) {
+    p[0] = v[0];
+  } else {
+    typedef float vec __attribute__((ext_vector_type(VX)));
+    vec w;
+#pragma unroll
+    for (int i = 0; i < VX; i++) w[i] = v[i];
+    *(vec *)p = w;
+  }
+}
+
 // Block barrier for LDS: the block's LDS accesses complete, then s_barrier.
 // __syncthreads also fences global memory, which waits for every load in
 // flight; the step kernels share nothing through global memory in a launch.
 __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
-}
-
-// ---- storage of wavefield levels: float, or FP16 with a power-of-two scale
-// per stored level (value = half * inv_scale).  Conversions saturate at the
-// FP16 range instead of overflowing.
-__device__ __forceinline__ float ld_level(const float *p, uint32_t o, float) {
-  return at(p, o);
-}
-__device__ __forceinline__ float ld_level(const __half *p, uint32_t o, float inv) {
-  return __half2float(at(p, o)) * inv;
-}
-__device__ __forceinline__ void st_level(float *p, uint32_t o, float v, float) {
-  at(p, o) = v;
-}
-__device__ __forceinline__ void st_level(__half *p, uint32_t o, float v, float scale) {
-  at(p, o) = __float2half_rn(fminf(fmaxf(v * scale, -65504.f), 65504.f));
 }
 
 // Scale for a level whose magnitude is at most bound: a power of two that
@@ -333,48 +394,81 @@ __device__ __forceinline__ float lam_inject(const RecMap &rm, int slot, int x, i
 
 struct CellArgs {
   int x, y, z;
-  uint32_t o;  // element offset of the cell
   float b;     // sponge factor (1 outside the sponge)
+  int rs;      // receiver slot of the plane, or -1 (then ri and rg are not set)
+  int ri;      // first receiver at the cell, or -1
+  float rg;    // what is injected there
 };
 
 __device__ __forceinline__ float sat_half(float v) { return fminf(fmaxf(v, -65504.f), 65504.f); }
+
+// ---- VX consecutive cells of a row (VX = 1, 2 or 4): the cells at plane
+// offset po (uniform) and lane offset o, in elements.  A lane's first cell is
+// at a multiple of VX (x tiles start at a multiple of it and nx is one), so
+// the accesses are naturally aligned.
+
+// stored words (T: uint16_t, uint32_t) at byte base b and byte offset o;
+// NT: the non-temporal hint, for inputs a launch reads once
+template <class T, int N, bool NT = false>
+__device__ __forceinline__ void ld_words(const char *b, uint32_t o, T (&u)[N]) {
+  if constexpr (N == 1) {
+    const T *q = (const T *)(b + (uint64_t)o);
+    u[0] = NT ? __builtin_nontemporal_load(q) : *q;
+  } else {
+    // (the instructions need no more than 4-byte alignment)
+    typedef T vec __attribute__((ext_vector_type(N), aligned(4)));
+    const vec *q = (const vec *)(b + (uint64_t)o);
+    const vec w = NT ? __builtin_nontemporal_load(q) : *q;
+#pragma unroll
+    for (int i = 0; i < N; i++) u[i] = w[i];
+  }
+}
+// N 32-bit words (1, 2 or 4)
+template <bool NT, int N>
+__device__ __forceinline__ void st_words(const char *b, uint32_t o, const uint32_t (&u)[N]) {
+  if constexpr (N == 1)
+    st_b32<NT>((void *)b, o, u[0]);
+  else if constexpr (N == 2)
+    st_b64<NT>((void *)b, o, (uint64_t)u[1] << 32 | u[0]);
+  else
+    st_b128<NT>((void *)b, o, make_uint4(u[0], u[1], u[2], u[3]));
+}
+__device__ __forceinline__ __half2 as_half2(uint32_t u) {
+  __half2 h;
+  __builtin_memcpy(&h, &u, 4);
+  return h;
+}
+__device__ __forceinline__ uint32_t half2_bits(float a, float b) {
+  const __half2 h = __floats2half2_rn(a, b);
+  uint32_t u;
+  __builtin_memcpy(&u, &h, 4);
+  return u;
+}
 
 // ---- Two FP16 fields stored as one __half2 per cell (first field in the
 // low half): one 4-byte load brings both, half the load instructions of two
 // separate FP16 arrays.  inv = 1/scale of each field.
 template <int VX>
-__device__ __forceinline__ void ld_pair(const __half2 *p, uint32_t o, const float (&inv)[2],
-                                        float (&v)[2][VX], uint32_t = 0) {
-  if constexpr (VX == 1) {
-    const __half2 w = at(p, o);
-    v[0][0] = __low2float(w) * inv[0];
-    v[1][0] = __high2float(w) * inv[1];
-  } else {
-    const uint2 u = at((const uint2 *)p, o >> 1);
-    __half2 a, b;
-    __builtin_memcpy(&a, &u.x, 4);
-    __builtin_memcpy(&b, &u.y, 4);
-    v[0][0] = __low2float(a) * inv[0];
-    v[1][0] = __high2float(a) * inv[1];
-    v[0][1] = __low2float(b) * inv[0];
-    v[1][1] = __high2float(b) * inv[1];
+__device__ __forceinline__ void ld_pair(const __half2 *p, uint32_t po, uint32_t o,
+                                        const float (&inv)[2], float (&v)[2][VX],
+                                        uint32_t = 0) {
+  uint32_t u[VX];
+  ld_words(adv(p, (uint64_t)po * 4u), o * 4u, u);
+#pragma unroll
+  for (int i = 0; i < VX; i++) {
+    v[0][i] = __low2float(as_half2(u[i])) * inv[0];
+    v[1][i] = __high2float(as_half2(u[i])) * inv[1];
   }
 }
 template <int VX, bool NT = true>
-__device__ __forceinline__ void st_pair(__half2 *p, uint32_t o, const float (&a)[VX],
-                                        const float (&b)[VX], const float (&scale)[2],
-                                        uint32_t = 0) {
-  const __half2 c0 = __floats2half2_rn(sat_half(a[0] * scale[0]), sat_half(b[0] * scale[1]));
-  uint32_t u0;
-  __builtin_memcpy(&u0, &c0, 4);
-  if constexpr (VX == 1) {
-    st_b32<NT>(p, o * 4u, u0);
-  } else {
-    const __half2 c1 = __floats2half2_rn(sat_half(a[1] * scale[0]), sat_half(b[1] * scale[1]));
-    uint32_t u1;
-    __builtin_memcpy(&u1, &c1, 4);
-    st_b64<NT>(p, o * 4u, (uint64_t)u1 << 32 | u0);
-  }
+__device__ __forceinline__ void st_pair(__half2 *p, uint32_t po, uint32_t o,
+                                        const float (&a)[VX], const float (&b)[VX],
+                                        const float (&scale)[2], uint32_t = 0) {
+  uint32_t u[VX];
+#pragma unroll
+  for (int i = 0; i < VX; i++)
+    u[i] = half2_bits(sat_half(a[i] * scale[0]), sat_half(b[i] * scale[1]));
+  st_words<NT>(adv(p, (uint64_t)po * 4u), o * 4u, u);
 }
 
 // ---- 24-bit storage: an FP32 value rounded to 24 bits per cell (sign, the
@@ -407,177 +501,220 @@ __device__ __forceinline__ float split_val(uint32_t hi, uint32_t lo) {
   return __uint_as_float(hi << 16 | (lo & 0xffu) << 8);
 }
 
-// VX = 2: two consecutive cells per lane (o even, n even: a pair of hi
-// values is 4-byte aligned, its lo bytes 2-byte aligned)
+// hi words of two cells a and b (a in the low half), and their lo bytes in
+// the two lowest bytes of a word
+__device__ __forceinline__ uint32_t split_hi(uint32_t qa, uint32_t qb) {
+  return qa >> 16 | (qb & 0xffff0000u);
+}
+__device__ __forceinline__ uint32_t split_lo(uint32_t qa, uint32_t qb) {
+  return (qa >> 8 & 0xffu) | (qb & 0xff00u);
+}
+// the two cells of hi word h whose lo bytes are the two lowest of l
+__device__ __forceinline__ void split_two(uint32_t h, uint32_t l, float &a, float &b) {
+  a = __uint_as_float(h << 16 | (l & 0xffu) << 8);
+  b = __uint_as_float((h & 0xffff0000u) | (l & 0xff00u));
+}
+
+// (n a multiple of VX: the lo bytes of VX cells are aligned to VX bytes)
 template <int VX>
-__device__ __forceinline__ void ld_vec(const Split *p, uint32_t o, float, float (&v)[VX],
-                                       uint32_t n) {
-  const char *b = (const char *)p;
+__device__ __forceinline__ void ld_vec(const Split *p, uint32_t po, uint32_t o, float,
+                                       float (&v)[VX], uint32_t n) {
+  const char *bh = adv(p, (uint64_t)po * 2u), *bl = adv(p, (uint64_t)n * 2u + po);
   if constexpr (VX == 1) {
-    const uint32_t hi = *(const unsigned short *)(b + o * 2u);
-    const uint32_t lo = *(const unsigned char *)(b + (2u * n + o));
-    v[0] = split_val(hi, lo);
+    v[0] = split_val(ldb<unsigned short>(bh, o * 2u), ldb<unsigned char>(bl, o));
   } else {
-    const uint32_t hi = *(const uint32_t *)(b + o * 2u);
-    const uint32_t lo = *(const unsigned short *)(b + (2u * n + o));
-    v[0] = __uint_as_float(hi << 16 | (lo & 0xffu) << 8);
-    v[1] = __uint_as_float((hi & 0xffff0000u) | (lo & 0xff00u));
+    uint32_t h[VX / 2], l;
+    ld_words(bh, o * 2u, h);
+    l = VX == 2 ? ldb<unsigned short>(bl, o) : ldb<uint32_t>(bl, o);
+    split_two(h[0], l, v[0], v[1]);
+    if constexpr (VX == 4) split_two(h[1], l >> 16, v[2], v[3]);
   }
 }
 template <int VX>
-__device__ __forceinline__ void ld_stream(const Split *p, uint32_t o, float inv,
+__device__ __forceinline__ void ld_stream(const Split *p, uint32_t po, uint32_t o, float inv,
                                           float (&v)[VX], uint32_t n) {
-  ld_vec<VX>(p, o, inv, v, n);
+  ld_vec<VX>(p, po, o, inv, v, n);
 }
 template <int VX, bool NT = true>
-__device__ __forceinline__ void st_vec(Split *p, uint32_t o, const float (&v)[VX], float,
-                                       uint32_t n) {
-  const uint32_t q0 = split_word(v[0]);
+__device__ __forceinline__ void st_vec(Split *p, uint32_t po, uint32_t o,
+                                       const float (&v)[VX], float, uint32_t n) {
+  const char *bh = adv(p, (uint64_t)po * 2u), *bl = adv(p, (uint64_t)n * 2u + po);
   if constexpr (VX == 1) {
-    st_b16<NT>(p, o * 2u, (unsigned short)(q0 >> 16));
-    st_b8<NT>(p, 2u * n + o, (unsigned char)(q0 >> 8));
+    const uint32_t q0 = split_word(v[0]);
+    st_b16<NT>((void *)bh, o * 2u, (unsigned short)(q0 >> 16));
+    st_b8<NT>((void *)bl, o, (unsigned char)(q0 >> 8));
   } else {
-    const uint32_t q1 = split_word(v[1]);
-    st_b32<NT>(p, o * 2u, q0 >> 16 | (q1 & 0xffff0000u));
-    st_b16<NT>(p, 2u * n + o, (unsigned short)((q0 >> 8 & 0xffu) | (q1 & 0xff00u)));
+    uint32_t h[VX / 2], l[VX / 2];
+#pragma unroll
+    for (int i = 0; i < VX / 2; i++) {
+      const uint32_t a = split_word(v[2 * i]), b = split_word(v[2 * i + 1]);
+      h[i] = split_hi(a, b);
+      l[i] = split_lo(a, b);
+    }
+    st_words<NT>(bh, o * 2u, h);
+    if constexpr (VX == 2)
+      st_b16<NT>((void *)bl, o, (unsigned short)l[0]);
+    else
+      st_b32<NT>((void *)bl, o, l[0] | l[1] << 16);
   }
 }
 // two fields stored together: first field in the low half of each pair
 template <int VX>
-__device__ __forceinline__ void ld_pair(const SplitPair *p, uint32_t o, const float (&)[2],
-                                        float (&v)[2][VX], uint32_t n) {
-  const char *b = (const char *)p;
+__device__ __forceinline__ void ld_pair(const SplitPair *p, uint32_t po, uint32_t o,
+                                        const float (&)[2], float (&v)[2][VX], uint32_t n) {
+  const char *bh = adv(p, (uint64_t)po * 4u), *bl = adv(p, (uint64_t)n * 4u + (uint64_t)po * 2u);
+  uint32_t h[VX];
+  ld_words(bh, o * 4u, h);
   if constexpr (VX == 1) {
-    const uint32_t hi = *(const uint32_t *)(b + o * 4u);
-    const uint32_t lo = *(const unsigned short *)(b + (4u * n + o * 2u));
-    v[0][0] = __uint_as_float(hi << 16 | (lo & 0xffu) << 8);
-    v[1][0] = __uint_as_float((hi & 0xffff0000u) | (lo & 0xff00u));
+    split_two(h[0], ldb<unsigned short>(bl, o * 2u), v[0][0], v[1][0]);
   } else {
-    const uint2 hi = *(const uint2 *)(b + o * 4u);
-    const uint32_t lo = *(const uint32_t *)(b + (4u * n + o * 2u));
-    v[0][0] = __uint_as_float(hi.x << 16 | (lo & 0xffu) << 8);
-    v[1][0] = __uint_as_float((hi.x & 0xffff0000u) | (lo & 0xff00u));
-    v[0][1] = __uint_as_float(hi.y << 16 | (lo >> 8 & 0xff00u));
-    v[1][1] = __uint_as_float((hi.y & 0xffff0000u) | (lo >> 16 & 0xff00u));
+    uint32_t l[VX / 2];
+    ld_words(bl, o * 2u, l);
+#pragma unroll
+    for (int i = 0; i < VX / 2; i++) {
+      split_two(h[2 * i], l[i], v[0][2 * i], v[1][2 * i]);
+      split_two(h[2 * i + 1], l[i] >> 16, v[0][2 * i + 1], v[1][2 * i + 1]);
+    }
   }
 }
 template <int VX, bool NT = true>
-__device__ __forceinline__ void st_pair(SplitPair *p, uint32_t o, const float (&a)[VX],
-                                        const float (&b)[VX], const float (&)[2],
-                                        uint32_t n) {
-  const uint32_t qa0 = split_word(a[0]), qb0 = split_word(b[0]);
-  const uint32_t h0 = qa0 >> 16 | (qb0 & 0xffff0000u);
-  const uint32_t l0 = (qa0 >> 8 & 0xffu) | (qb0 & 0xff00u);
+__device__ __forceinline__ void st_pair(SplitPair *p, uint32_t po, uint32_t o,
+                                        const float (&a)[VX], const float (&b)[VX],
+                                        const float (&)[2], uint32_t n) {
+  const char *bh = adv(p, (uint64_t)po * 4u), *bl = adv(p, (uint64_t)n * 4u + (uint64_t)po * 2u);
+  uint32_t h[VX], l[VX];
+#pragma unroll
+  for (int i = 0; i < VX; i++) {
+    const uint32_t qa = split_word(a[i]), qb = split_word(b[i]);
+    h[i] = split_hi(qa, qb);
+    l[i] = split_lo(qa, qb);
+  }
+  st_words<NT>(bh, o * 4u, h);
   if constexpr (VX == 1) {
-    st_b32<NT>(p, o * 4u, h0);
-    st_b16<NT>(p, 4u * n + o * 2u, (unsigned short)l0);
+    st_b16<NT>((void *)bl, o * 2u, (unsigned short)l[0]);
   } else {
-    const uint32_t qa1 = split_word(a[1]), qb1 = split_word(b[1]);
-    const uint32_t h1 = qa1 >> 16 | (qb1 & 0xffff0000u);
-    const uint32_t l1 = (qa1 >> 8 & 0xffu) | (qb1 & 0xff00u);
-    st_b64<NT>(p, o * 4u, (uint64_t)h1 << 32 | h0);
-    st_b32<NT>(p, 4u * n + o * 2u, l0 | l1 << 16);
+    uint32_t w[VX / 2];
+#pragma unroll
+    for (int i = 0; i < VX / 2; i++) w[i] = l[2 * i] | l[2 * i + 1] << 16;
+    st_words<NT>(bl, o * 2u, w);
   }
 }
 
-// ---- VX consecutive cells of a row (VX = 1 or 2).  A pair starts at an
-// even element offset (x tiles start at even x and nx is even when VX = 2),
-// so float2 / __half2 accesses are naturally aligned.
-template <int VX>
-__device__ __forceinline__ void ld_vec(const float *p, uint32_t o, float, float (&v)[VX],
-                                       uint32_t = 0) {
-  if constexpr (VX == 1) {
-    v[0] = at(p, o);
-  } else {
-    const float2 w = at((const float2 *)p, o >> 1);
-    v[0] = w.x;
-    v[1] = w.y;
-  }
+// ---- one field per array, FP32 or FP16
+template <int VX, bool NT = false>
+__device__ __forceinline__ void ld_vec(const float *p, uint32_t po, uint32_t o, float,
+                                       float (&v)[VX], uint32_t = 0) {
+  uint32_t u[VX];
+  ld_words<uint32_t, VX, NT>(adv(p, (uint64_t)po * 4u), o * 4u, u);
+#pragma unroll
+  for (int i = 0; i < VX; i++) v[i] = __uint_as_float(u[i]);
 }
 template <int VX>
-__device__ __forceinline__ void ld_vec(const __half *p, uint32_t o, float inv,
+__device__ __forceinline__ void ld_vec(const __half *p, uint32_t po, uint32_t o, float inv,
                                        float (&v)[VX], uint32_t = 0) {
+  const char *b = adv(p, (uint64_t)po * 2u);
   if constexpr (VX == 1) {
-    v[0] = __half2float(at(p, o)) * inv;
+    v[0] = __half2float(ldb<__half>(b, o * 2u)) * inv;
   } else {
-    const __half2 w = at((const __half2 *)p, o >> 1);
-    v[0] = __low2float(w) * inv;
-    v[1] = __high2float(w) * inv;
+    uint32_t u[VX / 2];
+    ld_words(b, o * 2u, u);
+#pragma unroll
+    for (int i = 0; i < VX / 2; i++) {
+      v[2 * i] = __low2float(as_half2(u[i])) * inv;
+      v[2 * i + 1] = __high2float(as_half2(u[i])) * inv;
+    }
   }
 }
 // The same loads with the non-temporal hint, for inputs a launch reads once
 // (the pointwise operands of a cell).
 template <int VX>
-__device__ __forceinline__ void ld_stream(const float *p, uint32_t o, float, float (&v)[VX],
-                                          uint32_t = 0) {
-  const float *q = (const float *)((const char *)p + (uint64_t)(o * 4u));
-  if constexpr (VX == 1) {
-    v[0] = __builtin_nontemporal_load(q);
-  } else {
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    const f2 w = __builtin_nontemporal_load((const f2 *)q);
-    v[0] = w.x;
-    v[1] = w.y;
-  }
+__device__ __forceinline__ void ld_stream(const float *p, uint32_t po, uint32_t o, float inv,
+                                          float (&v)[VX], uint32_t = 0) {
+  ld_vec<VX, true>(p, po, o, inv, v);
 }
 // FP16 levels keep the plain loads: with the hint the FP16 adjoint-state
 // and background steps ran 15-20 % slower (304^3, 2- and 4-byte lanes).
 template <int VX>
-__device__ __forceinline__ void ld_stream(const __half *p, uint32_t o, float inv,
+__device__ __forceinline__ void ld_stream(const __half *p, uint32_t po, uint32_t o, float inv,
                                           float (&v)[VX], uint32_t = 0) {
-  ld_vec<VX>(p, o, inv, v);
+  ld_vec<VX>(p, po, o, inv, v);
 }
-
-template <int VX, bool NT = true>
-__device__ __forceinline__ void st_vec(float *p, uint32_t o, const float (&v)[VX], float,
-                                       uint32_t = 0) {
-  if constexpr (VX == 1)
-    st_b32<NT>(p, o * 4u, __float_as_uint(v[0]));
-  else
-    st_b64<NT>(p, o * 4u, (uint64_t)__float_as_uint(v[1]) << 32 | __float_as_uint(v[0]));
-}
-template <int VX, bool NT = true>
-__device__ __forceinline__ void st_vec(__half *p, uint32_t o, const float (&v)[VX],
-                                       float scale, uint32_t = 0) {
-  if constexpr (VX == 1) {
-    st_b16<NT>(p, o * 2u, __half_as_ushort(__float2half_rn(sat_half(v[0] * scale))));
-  } else {
-    const __half2 c = __floats2half2_rn(sat_half(v[0] * scale), sat_half(v[1] * scale));
-    uint32_t u;
-    __builtin_memcpy(&u, &c, 4);
-    st_b32<NT>(p, o * 2u, u);
+// two FP32 fields interleaved cell by cell (non-temporal)
+template <int VX>
+__device__ __forceinline__ void ld_stream2(const float2 *p, uint32_t po, uint32_t o,
+                                           float (&a)[VX], float (&b)[VX]) {
+  const char *q = adv(p, (uint64_t)po * 8u);
+#pragma unroll
+  for (int h = 0; h < (VX + 1) / 2; h++) {
+    constexpr int N = VX == 1 ? 2 : 4;
+    uint32_t u[N];
+    ld_words<uint32_t, N, true>(q + 16 * h, o * 8u, u);
+#pragma unroll
+    for (int i = 0; i < N / 2; i++) {
+      a[2 * h + i] = __uint_as_float(u[2 * i]);
+      b[2 * h + i] = __uint_as_float(u[2 * i + 1]);
+    }
   }
 }
 
-// Generic z-marching leapfrog tile.  VX cells per lane along x (a tile is
-// 64*VX x RY*WY cells).  Op supplies (all const):
+template <int VX, bool NT = true>
+__device__ __forceinline__ void st_vec(float *p, uint32_t po, uint32_t o, const float (&v)[VX],
+                                       float, uint32_t = 0) {
+  uint32_t u[VX];
+#pragma unroll
+  for (int i = 0; i < VX; i++) u[i] = __float_as_uint(v[i]);
+  st_words<NT>(adv(p, (uint64_t)po * 4u), o * 4u, u);
+}
+template <int VX, bool NT = true>
+__device__ __forceinline__ void st_vec(__half *p, uint32_t po, uint32_t o,
+                                       const float (&v)[VX], float scale, uint32_t = 0) {
+  const char *b = adv(p, (uint64_t)po * 2u);
+  if constexpr (VX == 1) {
+    st_b16<NT>((void *)b, o * 2u, __half_as_ushort(__float2half_rn(sat_half(v[0] * scale))));
+  } else {
+    uint32_t u[VX / 2];
+#pragma unroll
+    for (int i = 0; i < VX / 2; i++)
+      u[i] = half2_bits(sat_half(v[2 * i] * scale), sat_half(v[2 * i + 1] * scale));
+    st_words<NT>(b, o * 2u, u);
+  }
+}
+
+// Generic z-marching leapfrog tile: LX*VX x RY*(64*WY/LX) cells of the xy
+// plane.  Op supplies (all const):
 //   static constexpr int NF, NPRE, NOUT, NMAX; static constexpr bool DAMP;
+//   static constexpr int REC;                   receivers: 0 none, 1 read, 2 injected
 //   Blk block(x0, x1, y0, y1, z0, z1);          uniform per-block state
 //   void first(const Blk&);                     (NMAX > 0) once per launch
-//   ldv<VX>(const Blk&, int f, uint32_t o, float (&v)[VX])   current level
-//   (PAIRED ops instead: ldv2<VX>(const Blk&, uint32_t o, float (&v)[NF][VX])
-//   loads every field of the current level at once)
+//   ldv<VX>(const Blk&, int f, uint32_t po, uint32_t o, float (&v)[VX])
+//     the current level at plane offset po and lane offset o
+//   (PAIRED ops instead: ldv2<VX>(const Blk&, uint32_t po, uint32_t o,
+//   float (&v)[NF][VX]) loads every field of the current level at once)
 //   Pln plane(const Blk&, int z);               uniform per-plane state
-//   prefetchv<VX>(const Blk&, float (&p)[NPRE][VX], uint32_t o)
+//   prefetchv<VX>(const Blk&, float (&p)[NPRE][VX], uint32_t po, uint32_t o)
+//   int rec_slot(const Pln&);                   (REC) receiver slot of the plane, or -1
+//   const int *rec_map(int slot);               (REC) its [ny][nx] first receivers
+//   float rec_value(int i);                     (REC 2) what receiver cell i injects
 //   void cell(const Blk&, const Pln&, const CellArgs&, const float *lap,
 //             const float *ctr, const float *pre, float (&out)[NOUT],
 //             float (&tmax)[NF]);                the new values of one cell
-//   storev<VX>(const Blk&, uint32_t o, const float (&out)[NOUT][VX])
+//   storev<VX>(const Blk&, uint32_t po, uint32_t o, const float (&out)[NOUT][VX])
 //   void publish_max(int f, float m);           (NMAX > 0) block max of |new|
 template <int B>
 struct StepSet {
   static constexpr int value = B;
 };
 
-template <class Op, int RY, int WY, int VX, int PZ, int LX, int D>
+template <class Op, int RY, int WY, int VX, int LX, int D>
 __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const Sponge &sp,
                                            const Op &op, const int L) {
   constexpr int NF = Op::NF;
   constexpr int NP = Op::NPRE > 0 ? Op::NPRE : 1;
   constexpr int NO = Op::NOUT;
-  // LX lanes per row (64: a wavefront per row; 32: two rows per wavefront),
-  // NG row groups per block
-  constexpr int NG = kTX * WY / LX;
+  // LX lanes per row (64: a wavefront per row; 32, 16, 8: it covers 2, 4, 8
+  // rows), NG row groups per block of NT threads
+  constexpr int NT = kTX * WY;
+  constexpr int NG = NT / LX;
   constexpr int TW = LX * VX;
   constexpr int TY = RY * NG;
   constexpr int LW = TW + 2 * kH;
@@ -588,15 +725,10 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
   // by two planes every second step (half the register moves), and the
   // pointwise inputs of the two steps sit in two buffers that the steps
   // refill alternately (no copy).
-  constexpr bool Q2 = Op::Q2 && D == 1 && PZ == 1;
+  constexpr bool Q2 = Op::Q2 && D == 1;
   constexpr int NB = Q2 ? 2 : D;  // buffer sets of loads in flight
-  // queue: planes z - kH .. z + kH + PZ - 1 (Q2: one more)
-  constexpr int NQ = 2 * kH + PZ + (Q2 ? 1 : 0);
-  // LDS planes form a ring of NR = kH + PZ slots (plane q in slot q % NR):
-  // a plane's halo is written when the plane enters the z queue as a lead,
-  // kH planes before its centre rows and its use
-  constexpr int NR = kH + PZ;
-  __shared__ __align__(16) float tile[NR][NF][LH][LW];
+  // queue: planes z - kH .. z + kH (Q2: one more)
+  constexpr int NQ = 2 * kH + 1 + (Q2 ? 1 : 0);
 
   const int bx = L % g.ntx;
   const int rest = L / g.ntx;
@@ -607,10 +739,19 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
   // x tiles start at the row start so that a wavefront's row maps onto whole
   // cache lines; the 4-cell shell at either end is masked
   const int x0 = bx * TW, y0 = kH + by * TY;
+  // The chunk's planes z0 .. z1 - 1.  Chunks are marched up and down in turn,
+  // so that two neighbours read the planes they share at about the same time,
+  // and a time loop turns every chunk round from one step to the next
+  // (g.back), so that a step starts with the planes the last one ended with.
+  // z is the count of a marched plane, zp its plane in the fields.
   const int z0 = kH + bz * g.zc;
   const int z1 = min(z0 + g.zc, g.nz - kH);
+  const bool down = ((bz & 1) ^ g.back) != 0;
+  const int zb = down ? z0 + z1 - 1 : 0, zs = down ? -1 : 1;
+  auto zp = [&](int z) { return zb + zs * z; };
+  auto zoff = [&](int z) { return (uint32_t)zp(z) * g.plane; };
   const int x = x0 + VX * tx;
-  const bool xin = x >= kH && x < g.nx - kH;  // with VX = 2 a pair is in or out
+  const bool xin = x >= kH && x < g.nx - kH;  // with VX > 1 a lane's cells are in or out
   const int xc = min(x, g.nx - VX);
 
   const auto blk = op.block(max(x0, kH), min(x0 + TW, g.nx - kH), y0,
@@ -618,6 +759,9 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
   if constexpr (Op::NMAX > 0)
     if (L == 0 && threadIdx.x == 0) op.first(blk);
 
+  // Cells are addressed by the plane's offset, uniform and added to the
+  // arrays' scalar base addresses, plus a lane's offset in the plane, which
+  // does not change over the march: no address arithmetic per plane.
   int yy[RY];
   bool in[RY];
   uint32_t row[RY];
@@ -632,20 +776,20 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
     for (int v = 0; v < VX; v++) bxy[j][v] = Op::DAMP ? fminf(sp.bx[xc + v], sp.by[yc]) : 1.f;
   }
 
-  // LDS halo in units of VX cells: 8 y-halo rows of 64 units and, per row,
+  // LDS halo in units of VX cells: 8 y-halo rows of LX units and, per row,
   // kH/VX units on either side, spread over the block's threads
   constexpr int XU = kH / VX;
   constexpr int NYH = 2 * kH * LX;
   constexpr int NXH = 2 * XU * TY;
   constexpr int NHALO = NYH + NXH;
-  constexpr int HPT = (NHALO + kTX * WY - 1) / (kTX * WY);
+  constexpr int HPT = (NHALO + NT - 1) / NT;
   uint32_t hoff[HPT];
-  short hr[HPT], hc[HPT];
+  short hr[HPT], hc[HPT], hs[HPT];
   bool hv[HPT];
 #pragma unroll
   for (int k = 0; k < HPT; k++) {
-    const int h = (int)threadIdx.x + k * kTX * WY;
-    hv[k] = h < NHALO;
+    const int h = (int)threadIdx.x + k * NT;
+    hv[k] = (k + 1) * NT <= NHALO || h < NHALO;
     int lr, lc;
     if (h < NYH) {  // rows 0..3 and TY+4..TY+7
       const int r = h / LX;
@@ -658,119 +802,115 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
       lc = c < XU ? VX * c : kH + TW + VX * (c - XU);
     }
     hr[k] = (short)lr;
+    hs[k] = (short)min(h, NHALO - 1);
     hc[k] = (short)lc;
     const int gy = min(max(y0 - kH + lr, 0), g.ny - 1);
     const int gx = min(max(x0 - kH + lc, 0), g.nx - VX);
     hoff[k] = (uint32_t)gy * g.nx + gx;
   }
 
-  // The tile marches PZ planes per step.  The loads of step z + D*PZ (queue
-  // leads, LDS halos, pointwise inputs) are issued before step z is computed:
-  // with D = 2 a load has two steps' compute to arrive, and the wait at a
-  // step's start leaves the previous step's loads in flight (the stores are
-  // invisible to the compiler's wait model and the barriers do not fence
-  // global memory, see st_b32 and lds_barrier).  Loads past the chunk's last
-  // step are clamped to planes the chunk reads anyway.
+  // The loads of step z + D (queue leads, LDS halos, pointwise inputs) are
+  // issued before step z is computed: with D = 2 a load has two steps'
+  // compute to arrive, and the wait at a step's start leaves the previous
+  // step's loads in flight (the stores are invisible to the compiler's wait
+  // model and the barriers do not fence global memory, see st_b32 and
+  // lds_barrier).  Loads past the chunk's last step are clamped to planes the
+  // chunk reads anyway.
   //
   // The LDS halo of a plane is loaded together with the plane's centre rows
   // (when the plane enters the z queue as a lead), not kH planes later: the
   // neighbouring tiles read those rows at about the same time, so they come
-  // from L2.  It waits in its LDS ring slot, not in registers; hl holds the
-  // halos of the leads in flight.
-  static_assert(D == 1 || PZ == 1, "a two-step lookahead takes one plane per step");
+  // from L2.  It waits kH planes in the loading thread's own place of stage
+  // (slot = plane mod kH), not in registers; hl holds the halos of the leads
+  // in flight.  tile holds the plane computed, in two buffers that the steps
+  // take in turn: a step writes one while slower wavefronts still read the
+  // other, so a step has a single barrier.
+  __shared__ __align__(16) float tile[2][NF][LH][LW];
+  __shared__ __align__(16) float stage[kH][NF][NHALO][VX];
   float q[NF][RY][VX][NQ];
-  float lead[NB][PZ][NF][RY][VX];
-  float hl[NB][PZ][NF][HPT][VX];
-  auto put_halo = [&](int slot, int f, int k, const float (&h)[VX]) {
-    float *d = &tile[slot][f][hr[k]][hc[k]];
-    if constexpr (VX == 1)
-      d[0] = h[0];
-    else
-      *(float2 *)d = make_float2(h[0], h[1]);
-  };
+  float lead[NB][NF][RY][VX];
+  float hl[NB][NF][HPT][VX];
   // pointwise inputs of the steps in flight, and of the step computed
-  float pre[NB][PZ][RY][NP][VX], cur[PZ][RY][NP][VX];
+  float pre[NB][RY][NP][VX], cur[RY][NP][VX];
   float tmax[NF];
-  // every field of the current level at element offset o
-  auto ld_all = [&](uint32_t o, float (&v)[NF][VX]) {
+  // every field of the current level at plane offset po, lane offset o
+  auto ld_all = [&](uint32_t po, uint32_t o, float (&v)[NF][VX]) {
     if constexpr (Op::PAIRED) {
-      op.template ldv2<VX>(blk, o, v);
+      op.template ldv2<VX>(blk, po, o, v);
     } else {
 #pragma unroll
-      for (int f = 0; f < NF; f++) op.template ldv<VX>(blk, f, o, v[f]);
+      for (int f = 0; f < NF; f++) op.template ldv<VX>(blk, f, po, o, v[f]);
     }
   };
   // the loads of the step at plane zs into buffer set b
   auto issue = [&](int zs, int b) {
+    const uint32_t zl = zoff(min(zs + kH, z1 - 1 + kH));
+    const uint32_t zn = zoff(min(zs, z1 - 1));
 #pragma unroll
-    for (int p = 0; p < PZ; p++) {
-      const uint32_t zl = (uint32_t)min(zs + kH + p, z1 - 1 + kH) * g.plane;
-      const uint32_t zn = (uint32_t)min(zs + p, z1 - 1) * g.plane;
+    for (int j = 0; j < RY; j++) {
+      float w[NF][VX];
+      ld_all(zl, row[j], w);
 #pragma unroll
-      for (int j = 0; j < RY; j++) {
-        float w[NF][VX];
-        ld_all(zl + row[j], w);
+      for (int f = 0; f < NF; f++)
 #pragma unroll
-        for (int f = 0; f < NF; f++)
-#pragma unroll
-          for (int v = 0; v < VX; v++) lead[b][p][f][j][v] = w[f][v];
-      }
-#pragma unroll
-      for (int k = 0; k < HPT; k++) {
-        float w[NF][VX];
-        ld_all(zl + hoff[k], w);
-#pragma unroll
-        for (int f = 0; f < NF; f++)
-#pragma unroll
-          for (int v = 0; v < VX; v++) hl[b][p][f][k][v] = w[f][v];
-      }
-#pragma unroll
-      for (int j = 0; j < RY; j++) op.template prefetchv<VX>(blk, pre[b][p][j], zn + row[j]);
+        for (int v = 0; v < VX; v++) lead[b][f][j][v] = w[f][v];
     }
+#pragma unroll
+    for (int k = 0; k < HPT; k++) {
+      float w[NF][VX];
+      ld_all(zl, hoff[k], w);
+#pragma unroll
+      for (int f = 0; f < NF; f++)
+#pragma unroll
+        for (int v = 0; v < VX; v++) hl[b][f][k][v] = w[f][v];
+    }
+#pragma unroll
+    for (int j = 0; j < RY; j++) op.template prefetchv<VX>(blk, pre[b][j], zn, row[j]);
   };
 #pragma unroll
   for (int f = 0; f < NF; f++) tmax[f] = 0.f;
+  // all of the chunk's first loads are in flight together
 #pragma unroll
   for (int j = 0; j < RY; j++) {
 #pragma unroll
     for (int k = 0; k < 2 * kH; k++) {
       float w[NF][VX];
-      ld_all((uint32_t)(z0 - kH + k) * g.plane + row[j], w);
+      ld_all(zoff(z0 - kH + k), row[j], w);
 #pragma unroll
       for (int f = 0; f < NF; f++)
 #pragma unroll
         for (int v = 0; v < VX; v++) q[f][j][v][k] = w[f][v];
     }
   }
+  {
+    float h[kH][HPT][NF][VX];
 #pragma unroll
-  for (int p = 0; p < kH; p++) {
+    for (int p = 0; p < kH; p++)
 #pragma unroll
-    for (int k = 0; k < HPT; k++) {
-      float h[NF][VX];
-      ld_all((uint32_t)(z0 + p) * g.plane + hoff[k], h);
+      for (int k = 0; k < HPT; k++) ld_all(zoff(z0 + p), hoff[k], h[p][k]);
 #pragma unroll
-      for (int f = 0; f < NF; f++)
-        if (hv[k]) put_halo((z0 + p) % NR, f, k, h[f]);
-    }
+    for (int b = 0; b < D; b++) issue(z0 + b, b);
+#pragma unroll
+    for (int p = 0; p < kH; p++)
+#pragma unroll
+      for (int k = 0; k < HPT; k++)
+#pragma unroll
+        for (int f = 0; f < NF; f++)
+          if (hv[k]) st_lds<VX>(stage[p][f][hs[k]], h[p][k][f]);
   }
-#pragma unroll
-  for (int b = 0; b < D; b++) issue(z0 + b * PZ, b);
 
   // The new values of a step are stored at the start of the next step,
   // after its wait and before its loads: the wait for a step's inputs then
   // finds stores and loads that were issued a whole step earlier.
-  float pend[PZ][RY][NO][VX];
+  float pend[RY][NO][VX];
   int pend_z = -1;
   auto flush = [&]() {
     if (pend_z >= 0) {
+      // (in a scalar register: the stores' base addresses have to be)
+      const uint32_t po = __builtin_amdgcn_readfirstlane(zoff(pend_z));
 #pragma unroll
-      for (int p = 0; p < PZ; p++)
-        if (pend_z + p < z1) {
-          const uint32_t po = (uint32_t)(pend_z + p) * g.plane;
-#pragma unroll
-          for (int j = 0; j < RY; j++)
-            if (in[j]) op.template storev<VX>(blk, po + row[j], pend[p][j]);
-        }
+      for (int j = 0; j < RY; j++)
+        if (in[j]) op.template storev<VX>(blk, po, row[j], pend[j]);
     }
   };
 
@@ -784,143 +924,146 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
     // the pointwise inputs are copied out of a buffer that this step's loads
     // refill
     constexpr bool COPY = bn == b;
-    float(&pw)[PZ][RY][NP][VX] = COPY ? cur : pre[b];
+    const int sl = (z - z0) % 2, ss = (z - z0) % kH;
+    // plane z to LDS: the centre rows from the queue, the halo from stage
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+#pragma unroll
+      for (int k = 0; k < HPT; k++) {
+        float h[VX];
+        ld_lds<VX>(stage[ss][f][hs[k]], h);
+        if (hv[k]) st_lds<VX>(&tile[sl][f][hr[k]][hc[k]], h);
+      }
+#pragma unroll
+      for (int j = 0; j < RY; j++) {
+        float c[VX];
+#pragma unroll
+        for (int v = 0; v < VX; v++) c[v] = q[f][j][v][kH + R];
+        st_lds<VX>(&tile[sl][f][kH + RY * ty + j][kH + VX * tx], c);
+      }
+    }
+    // the loads of this step: leads to the queue, their halo to stage
+    float(&pw)[RY][NP][VX] = COPY ? cur : pre[b];
     if constexpr (COPY) {
 #pragma unroll
-      for (int p = 0; p < PZ; p++)
+      for (int j = 0; j < RY; j++)
 #pragma unroll
-        for (int j = 0; j < RY; j++)
+        for (int k = 0; k < NP; k++)
 #pragma unroll
-          for (int k = 0; k < NP; k++)
-#pragma unroll
-            for (int v = 0; v < VX; v++) cur[p][j][k][v] = pre[b][p][j][k][v];
+          for (int v = 0; v < VX; v++) cur[j][k][v] = pre[b][j][k][v];
     }
 #pragma unroll
     for (int f = 0; f < NF; f++) {
 #pragma unroll
-      for (int j = 0; j < RY; j++) {
+      for (int j = 0; j < RY; j++)
 #pragma unroll
-        for (int p = 0; p < PZ; p++)
+        for (int v = 0; v < VX; v++) q[f][j][v][2 * kH + R] = lead[b][f][j][v];
 #pragma unroll
-          for (int v = 0; v < VX; v++) q[f][j][v][2 * kH + p + R] = lead[b][p][f][j][v];
-#pragma unroll
-        for (int p = 0; p < PZ; p++) {
-          float *d = &tile[(z + p) % NR][f][kH + RY * ty + j][kH + VX * tx];
-          if constexpr (VX == 1)
-            d[0] = q[f][j][0][kH + p + R];
-          else
-            *(float2 *)d = make_float2(q[f][j][0][kH + p + R], q[f][j][1][kH + p + R]);
-        }
-      }
-#pragma unroll
-      for (int p = 0; p < PZ; p++)
-#pragma unroll
-        for (int k = 0; k < HPT; k++)
-          if (hv[k]) put_halo((z + kH + p) % NR, f, k, hl[b][p][f][k]);
+      for (int k = 0; k < HPT; k++)
+        if (hv[k]) st_lds<VX>(stage[ss][f][hs[k]], hl[b][f][k]);
     }
     flush();
-    issue(z + D * PZ, bn);
+    issue(z + D, bn);
     lds_barrier();
+    const auto pl = op.plane(blk, zp(z));
+    const float bzv = Op::DAMP ? ldc(sp.bz, zp(z)) : 1.f;
+    // the receivers of the cells of a plane that has some (rs >= 0), loaded
+    // while the Laplacians are computed; not set on the other planes
+    int ri[RY][VX];
+    float rg[RY][VX];
+    int rs = -1;
+    if constexpr (Op::REC > 0) {
+      rs = op.rec_slot(pl);
+      if (rs >= 0) {
+        const int *rmap = op.rec_map(rs);
 #pragma unroll
-    for (int p = 0; p < PZ; p++) {
-      const int zz = z + p;
-      if (PZ > 1 && zz >= z1) break;
-      const int sl = zz % NR;
-      const uint32_t zo = (uint32_t)zz * g.plane;
-      const auto pl = op.plane(blk, zz);
-      const float bzv = Op::DAMP ? ldc(sp.bz, zz) : 1.f;
-      // Laplacians field by field.  The column above and below this
-      // thread's RY consecutive rows is read from LDS once per field (kH
-      // rows either side; the thread's own rows come from its z queues) and
-      // shared by the RY cells.
-      const int lr0 = kH + RY * ty, lc = kH + VX * tx;
-      float lap[RY][VX][NF];
+        for (int j = 0; j < RY; j++) ld_words<int, VX>((const char *)rmap, row[j] * 4u, ri[j]);
+        if constexpr (Op::REC == 2) {
 #pragma unroll
-      for (int f = 0; f < NF; f++) {
-        float col[RY + 2 * kH][VX];
+          for (int j = 0; j < RY; j++)
 #pragma unroll
-        for (int i = 0; i < kH; i++) {
-          const int ra = lr0 - kH + i, rb = lr0 + RY + i;
-          if constexpr (VX == 1) {
-            col[i][0] = tile[sl][f][ra][lc];
-            col[kH + RY + i][0] = tile[sl][f][rb][lc];
-          } else {
-            const float2 a2 = *(const float2 *)&tile[sl][f][ra][lc];
-            const float2 b2 = *(const float2 *)&tile[sl][f][rb][lc];
-            col[i][0] = a2.x;
-            col[i][1] = a2.y;
-            col[kH + RY + i][0] = b2.x;
-            col[kH + RY + i][1] = b2.y;
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < RY; j++)
-#pragma unroll
-          for (int v = 0; v < VX; v++) col[kH + j][v] = q[f][j][v][kH + p + R];
-#pragma unroll
-        for (int j = 0; j < RY; j++) {
-          if (!in[j]) continue;
-          // the row from lc - 4 to lc + VX + 3
-          const int lr = lr0 + j;
-          float xs[2 * kH + VX];
-          if constexpr (VX == 1) {
-#pragma unroll
-            for (int i = 0; i < 2 * kH + 1; i++) xs[i] = tile[sl][f][lr][lc - kH + i];
-          } else {
-#pragma unroll
-            for (int i = 0; i < kH + 1; i++) {
-              const float2 w = *(const float2 *)&tile[sl][f][lr][lc - kH + 2 * i];
-              xs[2 * i] = w.x;
-              xs[2 * i + 1] = w.y;
-            }
-          }
-#pragma unroll
-          for (int v = 0; v < VX; v++) {
-            // centre, then the x, y and z pairs, each pair summed first
-            float a = mul_r(t.c0, q[f][j][v][kH + p + R]);
-#pragma unroll
-            for (int k = 1; k <= kH; k++)
-              a = fma_r(t.cx[k - 1], add_r(xs[kH + v - k], xs[kH + v + k]), a);
-#pragma unroll
-            for (int k = 1; k <= kH; k++)
-              a = fma_r(t.cy[k - 1], add_r(col[kH + j - k][v], col[kH + j + k][v]), a);
-#pragma unroll
-            for (int k = 1; k <= kH; k++)
-              a = fma_r(t.cz[k - 1],
-                        add_r(q[f][j][v][kH + p - k + R], q[f][j][v][kH + p + k + R]), a);
-            lap[j][v][f] = a;
-          }
+            for (int v = 0; v < VX; v++) rg[j][v] = op.rec_value(max(ri[j][v], 0));
         }
       }
+    }
+    // Laplacians field by field.  The column above and below this
+    // thread's RY consecutive rows is read from LDS once per field (kH
+    // rows either side; the thread's own rows come from its z queues) and
+    // shared by the RY cells.
+    const int lr0 = kH + RY * ty, lc = kH + VX * tx;
+    float lap[RY][VX][NF];
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+      float col[RY + 2 * kH][VX];
+#pragma unroll
+      for (int i = 0; i < kH; i++) {
+        ld_lds<VX>(&tile[sl][f][lr0 - kH + i][lc], col[i]);
+        ld_lds<VX>(&tile[sl][f][lr0 + RY + i][lc], col[kH + RY + i]);
+      }
+#pragma unroll
+      for (int j = 0; j < RY; j++)
+#pragma unroll
+        for (int v = 0; v < VX; v++) col[kH + j][v] = q[f][j][v][kH + R];
 #pragma unroll
       for (int j = 0; j < RY; j++) {
-        if (!in[j]) continue;
-        float ctr[VX][NF];
+        // the row from lc - 4 to lc + VX + 3
+        float xs[2 * kH + VX];
 #pragma unroll
-        for (int f = 0; f < NF; f++)
+        for (int i = 0; i < kH; i += VX) {
+          float w[VX];
+          ld_lds<VX>(&tile[sl][f][lr0 + j][lc - kH + i], w);
 #pragma unroll
-          for (int v = 0; v < VX; v++) ctr[v][f] = q[f][j][v][kH + p + R];
+          for (int v = 0; v < VX; v++) xs[i + v] = w[v];
+          ld_lds<VX>(&tile[sl][f][lr0 + j][lc + VX + i], w);
+#pragma unroll
+          for (int v = 0; v < VX; v++) xs[kH + VX + i + v] = w[v];
+        }
+#pragma unroll
+        for (int v = 0; v < VX; v++) xs[kH + v] = q[f][j][v][kH + R];
 #pragma unroll
         for (int v = 0; v < VX; v++) {
-          CellArgs c;
-          c.x = x + v;
-          c.y = yy[j];
-          c.z = zz;
-          c.o = zo + row[j] + v;
-          c.b = fminf(bxy[j][v], bzv);
-          float pv[NP], o[NO];
+          // centre, then the x, y and z pairs, each pair summed first
+          float a = mul_r(t.c0, q[f][j][v][kH + R]);
 #pragma unroll
-          for (int k = 0; k < NP; k++) pv[k] = pw[p][j][k][v];
-          op.cell(blk, pl, c, lap[j][v], ctr[v], pv, o, tmax);
+          for (int k = 1; k <= kH; k++)
+            a = fma_r(t.cx[k - 1], add_r(xs[kH + v - k], xs[kH + v + k]), a);
 #pragma unroll
-          for (int k = 0; k < NO; k++) pend[p][j][k][v] = o[k];
+          for (int k = 1; k <= kH; k++)
+            a = fma_r(t.cy[k - 1], add_r(col[kH + j - k][v], col[kH + j + k][v]), a);
+#pragma unroll
+          for (int k = 1; k <= kH; k++)
+            a = fma_r(t.cz[k - 1], add_r(q[f][j][v][kH - k + R], q[f][j][v][kH + k + R]), a);
+          lap[j][v][f] = a;
         }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < RY; j++) {
+      if (!in[j]) continue;
+#pragma unroll
+      for (int v = 0; v < VX; v++) {
+        float ctr[NF];
+#pragma unroll
+        for (int f = 0; f < NF; f++) ctr[f] = q[f][j][v][kH + R];
+        CellArgs c;
+        c.x = x + v;
+        c.y = yy[j];
+        c.z = zp(z);
+        c.b = fminf(bxy[j][v], bzv);
+        c.rs = rs;
+        if constexpr (Op::REC > 0) c.ri = ri[j][v];
+        if constexpr (Op::REC == 2) c.rg = rg[j][v];
+        float pv[NP], o[NO];
+#pragma unroll
+        for (int k = 0; k < NP; k++) pv[k] = pw[j][k][v];
+        op.cell(blk, pl, c, lap[j][v], ctr, pv, o, tmax);
+#pragma unroll
+        for (int k = 0; k < NO; k++) pend[j][k][v] = o[k];
       }
     }
     pend_z = z;
-    lds_barrier();
-    // the queue moves by PZ planes a step, or by two after a Q2 pair
-    constexpr int MV = Q2 ? (R == 1 ? 2 : 0) : PZ;
+    // the queue moves by a plane a step, or by two after a Q2 pair
+    constexpr int MV = Q2 ? (R == 1 ? 2 : 0) : 1;
     if constexpr (MV > 0) {
 #pragma unroll
       for (int f = 0; f < NF; f++)
@@ -940,11 +1083,11 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
       step(z + 1, StepSet<1>{}, StepSet<1>{});
     }
   } else {
-    for (int z = z0; z < z1; z += D * PZ) {
+    for (int z = z0; z < z1; z += D) {
       step(z, StepSet<0>{}, StepSet<0>{});
       if constexpr (D == 2) {
-        if (z + PZ >= z1) break;
-        step(z + PZ, StepSet<1>{}, StepSet<0>{});
+        if (z + 1 >= z1) break;
+        step(z + 1, StepSet<1>{}, StepSet<0>{});
       }
     }
   }
@@ -974,7 +1117,7 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
 template <class Op, int RY, int WY, int VX, int LA, int LX>
 __global__ void __launch_bounds__(kTX *WY)
     march_kernel(const Grid g, const Taps t, const Sponge sp, const Op op) {
-  march_tile<Op, RY, WY, VX, 1, LX, LA>(g, t, sp, op,
+  march_tile<Op, RY, WY, VX, LX, LA>(g, t, sp, op,
                                         xcd_remap((int)blockIdx.x, (int)gridDim.x));
 }
 
@@ -984,6 +1127,7 @@ constexpr int kMaxBatch = 64;
 struct BatchTiles {
   int n;
   int zc;
+  int back;  // Grid::back of every shot
   int tile0[kMaxBatch + 1];
 };
 
@@ -994,6 +1138,7 @@ __host__ __device__ inline Grid tile_grid(int nx, int ny, int nz, int tw, int ty
   g.ny = ny;
   g.nz = nz;
   g.plane = (uint32_t)nx * ny;
+  g.back = 0;
   g.ntx = (nx - kH + tw - 1) / tw;
   g.nty = (ny - 2 * kH + ty - 1) / ty;
   g.zc = zc;
@@ -1010,8 +1155,9 @@ __global__ void __launch_bounds__(kTX *WY)
   const int Lg = xcd_remap((int)blockIdx.x, (int)gridDim.x);
   int s = 0;
   while (s + 1 < bt.n && Lg >= bt.tile0[s + 1]) s++;
-  const auto sh = bop.shot(s, LX * VX, RY * (kTX * WY / LX), bt.zc);
-  march_tile<typename BOp::Op, RY, WY, VX, 1, LX, LA>(sh.g, t, sh.sp, sh.op, Lg - bt.tile0[s]);
+  auto sh = bop.shot(s, LX * VX, RY * (kTX * WY / LX), bt.zc);
+  sh.g.back = bt.back;
+  march_tile<typename BOp::Op, RY, WY, VX, LX, LA>(sh.g, t, sh.sp, sh.op, Lg - bt.tile0[s]);
 }
 
 }  // namespace born

@@ -18,8 +18,7 @@ hipError_t launch_radj_step(const Geometry &geo, const Tune &tu, const RadjStep 
   op.vel1 = a.vel1; op.vel2 = a.vel2; op.img = a.img;
   op.s_prop = a.s_prop; op.r_prop = a.r_prop;
   op.pts = to_points(a.src); op.amp_pre = a.amp_pre; op.pre = a.pre;
-  op.rm = a.rec; op.tr = a.tr; op.tab = a.tab; op.sc = a.sc;
-  op.id = a.id; op.inject = a.inject; op.nx = geo.nx; op.ny = geo.ny;
+  op.rm = a.rec; op.gin = a.gin; op.nx = geo.nx; op.ny = geo.ny;
   return launch(geo, tu, op, st);
 }
 

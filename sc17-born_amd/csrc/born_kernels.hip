@@ -75,6 +75,68 @@ __global__ void src_amp_kernel(float *amp, int nsteps, int npts, const float *sr
   amp[(long long)s * stride + i] = a;
 }
 
+// The receivers of a window of steps (RecWindow): one thread per receiver
+// and trace sample j adds, in the order of the steps, what every step whose
+// eight samples id .. id + 7 hold j leaves there.
+__global__ void rec_accum_kernel(const RecWindow w, float *tr, const float *rv) {
+  const int s = blockIdx.z;
+  int nrec = w.nrec;
+  const int *rfirst = w.rfirst;
+  if (w.desc) {
+    const ShotDesc &d = w.desc[s];
+    nrec = d.nrec;
+    rfirst += d.rnext0;
+    rv += d.rnext0;
+    tr += d.tr0;
+  }
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int j = w.it0 / w.jt + (int)blockIdx.y;
+  if (i >= nrec || j >= w.ntb) return;
+  const int it1 = w.it0 + w.n - 1;
+  const int lo = max(w.it0, (j - 7) * w.jt), hi = min(it1, j * w.jt + w.jt - 1);
+  if (lo > hi) return;
+  const int c = rfirst[i];
+  float v = tr[(long long)j * nrec + i];
+  for (int it = lo; it <= hi; it++) {
+    const int id = it / w.jt, ii = it - id * w.jt;
+    if (id + 7 < w.ntb)
+      v = add_r(v, mul_r(rv[(long long)(it - w.it0) * w.stride + c], w.tab[ii * 8 + j - id]));
+  }
+  tr[(long long)j * nrec + i] = v;
+}
+
+// One thread per receiver and step of the window.
+__global__ void rec_inject_kernel(const RecWindow w, const float *tr, float *gin, int sum,
+                                  float scale) {
+  const int s = blockIdx.z;
+  int nrec = w.nrec;
+  const int *rfirst = w.rfirst, *rnext = w.rnext;
+  if (w.desc) {
+    const ShotDesc &d = w.desc[s];
+    nrec = d.nrec;
+    rfirst += d.rnext0;
+    rnext += d.rnext0;
+    gin += d.rnext0;
+    tr += d.tr0;
+  }
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nrec) return;
+  const int it = w.it0 + (int)blockIdx.y;
+  const int id = it / w.jt, ii = it - id * w.jt;
+  if (id + 7 >= w.ntb) return;
+  const float *t = w.tab + (long long)ii * 8;
+  float g;
+  if (sum) {
+    if (rfirst[i] != i) return;
+    g = 0.f;
+    for (int k = i; k >= 0; k = rnext[k])
+      g = add_r(g, sinc8(t, tr + (long long)id * nrec + k, nrec));
+  } else {
+    g = mul_r(scale, sinc8(t, tr + (long long)id * nrec + i, nrec));
+  }
+  gin[(long long)(it - w.it0) * w.stride + i] = g;
+}
+
 // out[i] += scale * acc[i] / (vel[i] * b[i]) on the interior.
 __global__ void adj_finish_kernel(float *out, const float *acc, const float *vel,
                                   const Sponge sp, int nx, int ny, int nz, float scale) {
@@ -111,7 +173,9 @@ __global__ void transpose_kernel(float *dst, const float *src, int n0, int n1) {
   {2, 4, 1, LA, 64}, {4, 4, 1, LA, 64}, {2, 8, 1, LA, 64}, {2, 16, 1, LA, 64},             \
       {1, 8, 1, LA, 64}, {1, 16, 1, LA, 64}, {1, 4, 2, LA, 32}, {2, 4, 2, LA, 32},         \
       {1, 8, 2, LA, 32}, {2, 8, 2, LA, 32}, {1, 12, 2, LA, 32}, {2, 2, 2, LA, 32}
-const TileShape kShapes[kNumShapes] = {BORN_TILES(1), BORN_TILES(2)};
+const TileShape kShapes[kNumShapes] = {
+    BORN_TILES(1),    BORN_TILES(2),    {1, 4, 4, 1, 16}, {1, 2, 4, 1, 16}, {2, 2, 4, 1, 16},
+    {1, 8, 4, 1, 16}, {1, 1, 4, 1, 8},  {1, 3, 4, 1, 8},  {1, 4, 4, 2, 16}, {1, 2, 4, 2, 16}};
 #undef BORN_TILES
 
 // the launchers of born_launch.h: dispatch on storage and scatter to the
@@ -196,6 +260,27 @@ hipError_t launch_interleave(float *dst, const float *a, const float *b, long lo
   if (nb > 65536) nb = 65536;
   hipLaunchKernelGGL(interleave_kernel, dim3((unsigned)nb), dim3(256), 0, st, (float2 *)dst, a,
                      b, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_rec_accum(const RecWindow &w, float *tr, const float *rv, hipStream_t st) {
+  if (w.n <= 0 || w.nrec <= 0) return hipSuccess;
+  // the samples of the window's steps
+  const int ns = (w.it0 + w.n - 1) / w.jt + 7 - w.it0 / w.jt + 1;
+  if (ns > 65535) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(rec_accum_kernel,
+                     dim3((w.nrec + 255) / 256, ns, w.desc ? w.nshots : 1), dim3(256), 0, st, w,
+                     tr, rv);
+  return hipGetLastError();
+}
+
+hipError_t launch_rec_inject(const RecWindow &w, const float *tr, float *gin, bool sum,
+                             float scale, hipStream_t st) {
+  if (w.n <= 0 || w.nrec <= 0) return hipSuccess;
+  if (w.n > 65535) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(rec_inject_kernel,
+                     dim3((w.nrec + 255) / 256, w.n, w.desc ? w.nshots : 1), dim3(256), 0, st,
+                     w, tr, gin, sum ? 1 : 0, scale);
   return hipGetLastError();
 }
 

@@ -16,19 +16,21 @@ struct Geometry {
 };
 
 // Tile shape: RY rows per thread, WY wavefronts per block, VX cells per lane
-// along x (VX = 2 needs an even nx), LA steps of load lookahead (1 or 2),
-// LX lanes per row (64, or 32: a wavefront covers two rows).  The tile is
+// along x (1, 2 or 4; nx a multiple of it), LA steps of load lookahead (1 or
+// 2), LX lanes per row (64, 32, 16 or 8: a wavefront covers 64 / LX rows).  The tile is
 // LX*VX x RY*(64*WY/LX) cells.
 struct TileShape {
   int ry, wy, vx, la, lx;
 };
-constexpr int kNumShapes = 24;
+constexpr int kNumShapes = 32;
 extern const TileShape kShapes[kNumShapes];
 
-// Launch configuration of one step kernel: tile shape and z planes per block.
+// Launch configuration of one step kernel: tile shape, z planes per block and
+// which way the z chunks are marched (Grid::back; see sweep() in born_abi.hip).
 struct Tune {
   int shape;
   int zchunk;
+  int back = 0;
 };
 
 // Source points: n entries of int4 (x, y, z, 0) in device memory.
@@ -57,9 +59,8 @@ struct FwdStep {
   SrcPts src;
   const float *amp;
   RecMap rec;
-  float *tr;
-  const float *tab;
-  int id, extract, scatter;
+  float *rv;  // [nrec] new r at the receiver cells, by first receiver (null: not wanted)
+  int scatter;
   Half h;
   float *rg;  // FP16 ring block: s ring at 0, r ring at 8, max |model| at 16
   float *hscale;
@@ -119,10 +120,7 @@ struct RadjStep {
   const float *amp_pre;
   int pre;
   RecMap rec;
-  const float *tr;
-  const float *tab;
-  float sc;
-  int id, inject;
+  const float *gin;  // [nrec] added to r by receiver (null: nothing)
 };
 
 struct SrecStep {
@@ -145,9 +143,7 @@ struct LamStep {
   const float *vel, *sig;
   float *acc;
   RecMap rec;
-  const float *tr;
-  const float *tab;
-  int id, inject;
+  const float *gin;  // [nrec] injected by the cell's first receiver (null: nothing)
   Half h;
   Ring ring;
   float inj;
@@ -230,6 +226,24 @@ hipError_t launch_srec_step(const Geometry &geo, const Tune &tu, const SrecStep 
                             hipStream_t st);
 hipError_t launch_lam_step(const Geometry &geo, const Tune &tu, const LamStep &a,
                            hipStream_t st);
+// Receivers of one shot, or of a batch (desc, nshots; nrec the most of a
+// shot): the steps [it0, it0 + n) of a time loop with jt steps per trace
+// sample, whose values are rows of `stride` floats in rv / gin.  rfirst[i]:
+// the first receiver at receiver i's cell.
+struct RecWindow {
+  int it0, n, jt, nrec, ntb;
+  long long stride;
+  const int *rfirst, *rnext;
+  const float *tab;  // [jt][8]
+  const ShotDesc *desc;
+  int nshots;
+};
+// traces (time-major) += the steps' samples: tr[id + k] += r tab[ii][k]
+hipError_t launch_rec_accum(const RecWindow &w, float *tr, const float *rv, hipStream_t st);
+// what the steps inject.  sum: by cell, the sum over its receivers of their
+// interpolated samples; else by receiver, scale times the sample
+hipError_t launch_rec_inject(const RecWindow &w, const float *tr, float *gin, bool sum,
+                             float scale, hipStream_t st);
 hipError_t launch_fill(float *p, long long n, float v, hipStream_t st);
 // dst (2n floats) = a and b interleaved cell by cell
 hipError_t launch_interleave(float *dst, const float *a, const float *b, long long n,

@@ -37,9 +37,8 @@ struct SrcPln {
   int slot;
 };
 
-__device__ __forceinline__ int rec_first(const RecMap &rm, int slot, int x, int y,
-                                         int nx, int ny) {
-  return rm.rmap[((long long)slot * ny + y) * nx + x];
+__device__ __forceinline__ const int *rec_plane(const RecMap &rm, int slot, int nx, int ny) {
+  return rm.rmap + (long long)slot * ny * nx;
 }
 
 // Scaled storage (FP16) shares the state of the ops (unused with float and
@@ -80,7 +79,7 @@ __device__ __forceinline__ float amp_sum(const Points &pts, const float *amp) {
 template <int SCATTER, class T, bool NT = true>
 struct FwdOp {
   static constexpr bool H = kScaled<T>;
-  static constexpr int NF = 2, NPRE = 4, NOUT = 3, NMAX = H ? 2 : 0;
+  static constexpr int NF = 2, NPRE = 4, NOUT = 3, NMAX = H ? 2 : 0, REC = 1;
   // FP16 and 24-bit levels hold s and r together per cell (sr1: level k,
   // sr0: level k-1, srn: level k+1, the same buffer as sr0 in place)
   static constexpr bool PAIRED = kNarrow<T>;
@@ -106,9 +105,8 @@ struct FwdOp {
   Points pts;
   const float *__restrict__ amp;  // source amplitudes of this step [npts]
   RecMap rm;
-  float *__restrict__ tr;  // traces, time-major [ntb][nrec]
-  const float *__restrict__ tab;
-  int id, extract, nx, ny;
+  float *rv;  // the new r at the receiver cells (nullptr: not wanted)
+  int nx, ny;
   uint32_t nlev;  // cells of a level (24-bit storage: the lo bytes follow the hi values)
   // FP16 scale state in as few scalar registers as possible (the loop needs
   // none of it, but kernel arguments stay live in scalar registers, and
@@ -157,62 +155,53 @@ struct FwdOp {
     atomicMax(&ring(f).maxb[slot(2)], __float_as_uint(m));
   }
   template <int VX>
-  __device__ void ldv(const Blk2 &b, int f, uint32_t o, float (&v)[VX]) const {
-    ld_vec<VX>(f == 0 ? s1 : r1, o, b.ic[f], v, nlev);
+  __device__ void ldv(const Blk2 &b, int f, uint32_t po, uint32_t o, float (&v)[VX]) const {
+    ld_vec<VX>(f == 0 ? s1 : r1, po, o, b.ic[f], v, nlev);
   }
   template <int VX>
-  __device__ void ldv2(const Blk2 &b, uint32_t o, float (&v)[2][VX]) const {
-    ld_pair<VX>(sr1, o, b.ic, v, nlev);
+  __device__ void ldv2(const Blk2 &b, uint32_t po, uint32_t o, float (&v)[2][VX]) const {
+    ld_pair<VX>(sr1, po, o, b.ic, v, nlev);
   }
   __device__ SrcPln plane(const Blk2 &b, int z) const {
     return {points_on_plane(pts, b.pb, z), ldc(rm.plane_slot, z)};
   }
+  __device__ int rec_slot(const SrcPln &pl) const { return rv ? pl.slot : -1; }
+  __device__ const int *rec_map(int slot) const { return rec_plane(rm, slot, nx, ny); }
   template <int VX>
-  __device__ void prefetchv(const Blk2 &b, float (&p)[NPRE][VX], uint32_t o) const {
+  __device__ void prefetchv(const Blk2 &b, float (&p)[NPRE][VX], uint32_t po,
+                            uint32_t o) const {
     if constexpr (PAIRED) {
       float sr[2][VX];
-      ld_pair<VX>(sr0, o, b.io, sr, nlev);
+      ld_pair<VX>(sr0, po, o, b.io, sr, nlev);
 #pragma unroll
       for (int v = 0; v < VX; v++) {
         p[0][v] = sr[0][v];
         p[1][v] = sr[1][v];
       }
     } else if constexpr (NT) {
-      ld_stream<VX>(s0, o, b.io[0], p[0], nlev);
-      ld_stream<VX>(r0, o, b.io[1], p[1], nlev);
+      ld_stream<VX>(s0, po, o, b.io[0], p[0], nlev);
+      ld_stream<VX>(r0, po, o, b.io[1], p[1], nlev);
     } else {
-      ld_vec<VX>(s0, o, b.io[0], p[0], nlev);
-      ld_vec<VX>(r0, o, b.io[1], p[1], nlev);
+      ld_vec<VX>(s0, po, o, b.io[0], p[0], nlev);
+      ld_vec<VX>(r0, po, o, b.io[1], p[1], nlev);
     }
     if constexpr (NT) {
-      const char *q = (const char *)vm + (uint64_t)o * 8u;
-      if constexpr (VX == 1) {
-        typedef float f2 __attribute__((ext_vector_type(2)));
-        const f2 w = __builtin_nontemporal_load((const f2 *)q);
-        p[2][0] = w.x;
-        p[3][0] = w.y;
-      } else {
-        typedef float f4 __attribute__((ext_vector_type(4)));
-        const f4 w = __builtin_nontemporal_load((const f4 *)q);
-        p[2][0] = w.x;
-        p[3][0] = w.y;
-        p[2][1] = w.z;
-        p[3][1] = w.w;
-      }
+      ld_stream2<VX>(vm, po, o, p[2], p[3]);
     } else {
-      ld_vec<VX>(vel, o, 1.f, p[2]);
-      ld_vec<VX>(model, o, 1.f, p[3]);
+      ld_vec<VX>(vel, po, o, 1.f, p[2]);
+      ld_vec<VX>(model, po, o, 1.f, p[3]);
     }
   }
   template <int VX>
-  __device__ void storev(const Blk2 &b, uint32_t o, const float (&out)[NOUT][VX]) const {
+  __device__ void storev(const Blk2 &b, uint32_t po, uint32_t o,
+                         const float (&out)[NOUT][VX]) const {
     if constexpr (PAIRED) {
-      st_pair<VX, NT>(srn, o, out[0], out[1], b.sn, nlev);
+      st_pair<VX, NT>(srn, po, o, out[0], out[1], b.sn, nlev);
     } else {
-      st_vec<VX, NT>(s_new, o, out[0], b.sn[0], nlev);
-      st_vec<VX, NT>(r0, o, out[1], b.sn[1], nlev);
+      st_vec<VX, NT>(s_new, po, o, out[0], b.sn[0], nlev);
+      st_vec<VX, NT>(r0, po, o, out[1], b.sn[1], nlev);
     }
-    if (hist) st_vec<VX, NT>(hist, o, out[2], b.sh, nlev);
+    if (hist) st_vec<VX, NT>(hist, po, o, out[2], b.sh, nlev);
   }
   __device__ void cell(const Blk2 &b, const SrcPln &pl, const CellArgs &c,
                        const float *lap, const float *ctr, const float *p,
@@ -238,25 +227,13 @@ struct FwdOp {
       tmax[0] = fmaxf(tmax[0], fabsf(sn));
       tmax[1] = fmaxf(tmax[1], fabsf(rn));
     }
-    if (pl.slot >= 0 && extract) {
-      // the 8 samples of a receiver are distinct, but the compiler cannot
-      // tell; all loads first, then all stores, one wait instead of eight
-      for (int i = rec_first(rm, pl.slot, c.x, c.y, nx, ny); i >= 0; i = rm.rnext[i]) {
-        float *q = tr + (long long)id * rm.nrec + i;
-        float v[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) v[k] = q[(long long)k * rm.nrec];
-#pragma unroll
-        for (int k = 0; k < 8; k++)
-          q[(long long)k * rm.nrec] = add_r(v[k], mul_r(rn, ldc(tab, k)));
-      }
-    }
+    if (c.rs >= 0 && c.ri >= 0) st_b32<false>(rv, (uint32_t)c.ri * 4u, __float_as_uint(rn));
   }
 };
 
 // ------------------------------------------------------------- sourceProp
 struct SrcOp {
-  static constexpr int NF = 1, NPRE = 2, NOUT = 1, NMAX = 0;
+  static constexpr int NF = 1, NPRE = 2, NOUT = 1, NMAX = 0, REC = 0;
   static constexpr bool PAIRED = false;
   static constexpr bool Q2 = false;
   static constexpr bool DAMP = false;
@@ -269,20 +246,22 @@ struct SrcOp {
     return points_in_block(pts, x0, x1, y0, y1, z0, z1);
   }
   template <int VX>
-  __device__ void ldv(uint32_t, int, uint32_t o, float (&v)[VX]) const {
-    ld_vec<VX>(s1, o, 1.f, v);
+  __device__ void ldv(uint32_t, int, uint32_t po, uint32_t o, float (&v)[VX]) const {
+    ld_vec<VX>(s1, po, o, 1.f, v);
   }
   __device__ uint32_t plane(uint32_t blk, int z) const {
     return points_on_plane(pts, blk, z);
   }
   template <int VX>
-  __device__ void prefetchv(uint32_t, float (&p)[NPRE][VX], uint32_t o) const {
-    ld_vec<VX>(s0, o, 1.f, p[0]);
-    ld_vec<VX>(vel, o, 1.f, p[1]);
+  __device__ void prefetchv(uint32_t, float (&p)[NPRE][VX], uint32_t po,
+                            uint32_t o) const {
+    ld_vec<VX>(s0, po, o, 1.f, p[0]);
+    ld_vec<VX>(vel, po, o, 1.f, p[1]);
   }
   template <int VX>
-  __device__ void storev(uint32_t, uint32_t o, const float (&out)[NOUT][VX]) const {
-    st_vec<VX>(s0, o, out[0], 1.f);
+  __device__ void storev(uint32_t, uint32_t po, uint32_t o,
+                         const float (&out)[NOUT][VX]) const {
+    st_vec<VX>(s0, po, o, out[0], 1.f);
   }
   __device__ void cell(uint32_t, uint32_t pm, const CellArgs &c, const float *lap,
                        const float *ctr, const float *p, float (&out)[NOUT],
@@ -295,7 +274,7 @@ struct SrcOp {
 
 // ------------------------------------------------------ reference adjoint
 struct RadjOp {
-  static constexpr int NF = 2, NPRE = 5, NOUT = 3, NMAX = 0;
+  static constexpr int NF = 2, NPRE = 5, NOUT = 3, NMAX = 0, REC = 2;
   static constexpr bool PAIRED = false;
   static constexpr bool Q2 = false;
   static constexpr bool DAMP = true;
@@ -313,34 +292,37 @@ struct RadjOp {
   const float *__restrict__ amp_pre;
   int pre;
   RecMap rm;
-  const float *__restrict__ tr;
-  const float *__restrict__ tab;
-  float sc;  // (float)dir / (float)jt
-  int id, inject, nx, ny;
+  const float *__restrict__ gin;  // injected per receiver (nullptr: nothing)
+  int nx, ny;
 
+  __device__ int rec_slot(const SrcPln &pl) const { return gin ? pl.slot : -1; }
+  __device__ const int *rec_map(int slot) const { return rec_plane(rm, slot, nx, ny); }
+  __device__ float rec_value(int i) const { return gin[i]; }
   __device__ uint32_t block(int x0, int x1, int y0, int y1, int z0, int z1) const {
     return pre ? points_in_block(pts, x0, x1, y0, y1, z0, z1) : 0u;
   }
   template <int VX>
-  __device__ void ldv(uint32_t, int f, uint32_t o, float (&v)[VX]) const {
-    ld_vec<VX>(f == 0 ? s1 : r1, o, 1.f, v);
+  __device__ void ldv(uint32_t, int f, uint32_t po, uint32_t o, float (&v)[VX]) const {
+    ld_vec<VX>(f == 0 ? s1 : r1, po, o, 1.f, v);
   }
   __device__ SrcPln plane(uint32_t blk, int z) const {
     return {points_on_plane(pts, blk, z), ldc(rm.plane_slot, z)};
   }
   template <int VX>
-  __device__ void prefetchv(uint32_t, float (&p)[NPRE][VX], uint32_t o) const {
-    ld_vec<VX>(s0, o, 1.f, p[0]);
-    ld_vec<VX>(r0, o, 1.f, p[1]);
-    ld_vec<VX>(vel1, o, 1.f, p[2]);
-    ld_vec<VX>(vel2, o, 1.f, p[3]);
-    ld_vec<VX>(img, o, 1.f, p[4]);
+  __device__ void prefetchv(uint32_t, float (&p)[NPRE][VX], uint32_t po,
+                            uint32_t o) const {
+    ld_vec<VX>(s0, po, o, 1.f, p[0]);
+    ld_vec<VX>(r0, po, o, 1.f, p[1]);
+    ld_vec<VX>(vel1, po, o, 1.f, p[2]);
+    ld_vec<VX>(vel2, po, o, 1.f, p[3]);
+    ld_vec<VX>(img, po, o, 1.f, p[4]);
   }
   template <int VX>
-  __device__ void storev(uint32_t, uint32_t o, const float (&out)[NOUT][VX]) const {
-    if (s_prop) st_vec<VX>(s0, o, out[0], 1.f);
-    st_vec<VX>(r0, o, out[1], 1.f);
-    st_vec<VX>(img, o, out[2], 1.f);
+  __device__ void storev(uint32_t, uint32_t po, uint32_t o,
+                         const float (&out)[NOUT][VX]) const {
+    if (s_prop) st_vec<VX>(s0, po, o, out[0], 1.f);
+    st_vec<VX>(r0, po, o, out[1], 1.f);
+    st_vec<VX>(img, po, o, out[2], 1.f);
   }
   __device__ void cell(uint32_t, const SrcPln &pl, const CellArgs &c, const float *lap,
                        const float *ctr, const float *p, float (&out)[NOUT],
@@ -355,9 +337,11 @@ struct RadjOp {
     }
     const float b = c.b;
     float rn = r_prop ? leap(b, p[3], lap[1], ctr[1], p[1]) : mul_r(b, mul_r(b, p[1]));
-    if (pl.slot >= 0 && inject) {
-      for (int i = rec_first(rm, pl.slot, c.x, c.y, nx, ny); i >= 0; i = rm.rnext[i])
-        rn = add_r(rn, mul_r(sc, sinc8(tab, tr + (long long)id * rm.nrec + i, rm.nrec)));
+    if (c.rs >= 0) {
+      // the receivers of a cell one after the other, as the reference adds them
+      if (c.ri >= 0) rn = add_r(rn, c.rg);
+      if (rm.shared && c.ri >= 0)
+        for (int i = rm.rnext[c.ri]; i >= 0; i = rm.rnext[i]) rn = add_r(rn, gin[i]);
     }
     out[0] = sn;
     out[1] = rn;
@@ -369,7 +353,7 @@ struct RadjOp {
 template <int SCATTER, class T>
 struct SrecOp {
   static constexpr bool H = kScaled<T>;
-  static constexpr int NF = 1, NPRE = 2, NOUT = 2, NMAX = H ? 1 : 0;
+  static constexpr int NF = 1, NPRE = 2, NOUT = 2, NMAX = H ? 1 : 0, REC = 0;
   static constexpr bool PAIRED = false;
   static constexpr bool Q2 = kNarrow<T>;  // steps in pairs (march_tile)
   static constexpr bool DAMP = true;
@@ -412,25 +396,27 @@ struct SrecOp {
     atomicMax(&ring.maxb[sl.nxt], __float_as_uint(m));
   }
   template <int VX>
-  __device__ void ldv(const Blk1 &b, int, uint32_t o, float (&v)[VX]) const {
-    ld_vec<VX>(s1, o, b.ic, v, nlev);
+  __device__ void ldv(const Blk1 &b, int, uint32_t po, uint32_t o, float (&v)[VX]) const {
+    ld_vec<VX>(s1, po, o, b.ic, v, nlev);
   }
   __device__ uint32_t plane(const Blk1 &b, int z) const {
     return points_on_plane(pts, b.pb, z);
   }
   template <int VX>
-  __device__ void prefetchv(const Blk1 &b, float (&p)[NPRE][VX], uint32_t o) const {
-    ld_stream<VX>(s0, o, b.io, p[0], nlev);
+  __device__ void prefetchv(const Blk1 &b, float (&p)[NPRE][VX], uint32_t po,
+                            uint32_t o) const {
+    ld_stream<VX>(s0, po, o, b.io, p[0], nlev);
     // FP32: the velocity without the hint (114 -> 103 us per step at 304^3)
     if constexpr (kNarrow<T>)
-      ld_stream<VX>(vel, o, 1.f, p[1]);
+      ld_stream<VX>(vel, po, o, 1.f, p[1]);
     else
-      ld_vec<VX>(vel, o, 1.f, p[1]);
+      ld_vec<VX>(vel, po, o, 1.f, p[1]);
   }
   template <int VX>
-  __device__ void storev(const Blk1 &b, uint32_t o, const float (&out)[NOUT][VX]) const {
-    st_vec<VX>(s_new, o, out[0], b.sn, nlev);
-    if (sig) st_vec<VX>(sig, o, out[1], b.sh, nlev);
+  __device__ void storev(const Blk1 &b, uint32_t po, uint32_t o,
+                         const float (&out)[NOUT][VX]) const {
+    st_vec<VX>(s_new, po, o, out[0], b.sn, nlev);
+    if (sig) st_vec<VX>(sig, po, o, out[1], b.sh, nlev);
   }
   __device__ void cell(const Blk1 &, uint32_t pm, const CellArgs &c, const float *lap,
                        const float *ctr, const float *p, float (&out)[NOUT],
@@ -450,7 +436,7 @@ struct SrecOp {
 template <class T>
 struct LamOp {
   static constexpr bool H = kScaled<T>;
-  static constexpr int NF = 1, NPRE = 4, NOUT = 2, NMAX = H ? 1 : 0;
+  static constexpr int NF = 1, NPRE = 4, NOUT = 2, NMAX = H ? 1 : 0, REC = 2;
   static constexpr bool PAIRED = false;
   static constexpr bool Q2 = kNarrow<T>;  // steps in pairs (march_tile)
   static constexpr bool DAMP = true;
@@ -460,9 +446,8 @@ struct LamOp {
   const T *__restrict__ sig;
   float *__restrict__ acc;
   RecMap rm;
-  const float *__restrict__ tr;
-  const float *__restrict__ tab;
-  int id, inject, nx, ny;
+  const float *__restrict__ gin;  // injected per receiver cell (nullptr: nothing)
+  int nx, ny;
   Ring ring;
   Slots sl;
   float gain;
@@ -479,7 +464,7 @@ struct LamOp {
       b.ic = 1.f / ring.scale[sl.cur];
       b.io = 1.f / ring.scale[sl.old];
       const float bu = gain * ring_max(ring, sl.cur) + ring_max(ring, sl.old) +
-                       (inject ? inj * __uint_as_float(*trmax) : 0.f);
+                       (gin ? inj * __uint_as_float(*trmax) : 0.f);
       b.sn = level_scale(bu);
       b.sh = 1.f / *hscale;
     }
@@ -493,36 +478,41 @@ struct LamOp {
     atomicMax(&ring.maxb[sl.nxt], __float_as_uint(m));
   }
   template <int VX>
-  __device__ void ldv(const Blk1 &b, int, uint32_t o, float (&v)[VX]) const {
-    ld_vec<VX>(u1, o, b.ic, v, nlev);
+  __device__ void ldv(const Blk1 &b, int, uint32_t po, uint32_t o, float (&v)[VX]) const {
+    ld_vec<VX>(u1, po, o, b.ic, v, nlev);
   }
   __device__ int plane(const Blk1 &, int z) const { return ldc(rm.plane_slot, z); }
+  __device__ int rec_slot(int slot) const { return gin ? slot : -1; }
+  __device__ const int *rec_map(int slot) const { return rec_plane(rm, slot, nx, ny); }
+  __device__ float rec_value(int i) const { return gin[i]; }
   template <int VX>
-  __device__ void prefetchv(const Blk1 &b, float (&p)[NPRE][VX], uint32_t o) const {
-    ld_stream<VX>(u0, o, b.io, p[0], nlev);
-    ld_stream<VX>(sig, o, b.sh, p[2], nlev);
+  __device__ void prefetchv(const Blk1 &b, float (&p)[NPRE][VX], uint32_t po,
+                            uint32_t o) const {
+    ld_stream<VX>(u0, po, o, b.io, p[0], nlev);
+    ld_stream<VX>(sig, po, o, b.sh, p[2], nlev);
     // FP32: velocity and image without the non-temporal hint (read, and the
     // image written, every step: 143 against 155 us per step at 304^3);
     // the FP16 step is faster with it
     if constexpr (kNarrow<T>) {
-      ld_stream<VX>(vel, o, 1.f, p[1]);
-      ld_stream<VX>(acc, o, 1.f, p[3]);
+      ld_stream<VX>(vel, po, o, 1.f, p[1]);
+      ld_stream<VX>(acc, po, o, 1.f, p[3]);
     } else {
-      ld_vec<VX>(vel, o, 1.f, p[1]);
-      ld_vec<VX>(acc, o, 1.f, p[3]);
+      ld_vec<VX>(vel, po, o, 1.f, p[1]);
+      ld_vec<VX>(acc, po, o, 1.f, p[3]);
     }
   }
   template <int VX>
-  __device__ void storev(const Blk1 &b, uint32_t o, const float (&out)[NOUT][VX]) const {
-    st_vec<VX>(u0, o, out[0], b.sn, nlev);
-    st_vec<VX, kNarrow<T>>(acc, o, out[1], 1.f);
+  __device__ void storev(const Blk1 &b, uint32_t po, uint32_t o,
+                         const float (&out)[NOUT][VX]) const {
+    st_vec<VX>(u0, po, o, out[0], b.sn, nlev);
+    st_vec<VX, kNarrow<T>>(acc, po, o, out[1], 1.f);
   }
   __device__ void cell(const Blk1 &, int slot, const CellArgs &c, const float *lap,
                        const float *ctr, const float *p, float (&out)[NOUT],
                        float (&tmax)[NF]) const {
     const float bb = c.b, v = p[1];
     float un = leap(bb, v, lap[0], ctr[0], p[0]);
-    if (slot >= 0 && inject) un = lam_inject(rm, slot, c.x, c.y, nx, ny, tr, tab, id, v, bb, un);
+    if (c.rs >= 0 && c.ri >= 0) un = fma_r(mul_r(v, bb), c.rg, un);
     if constexpr (H) tmax[0] = fmaxf(tmax[0], fabsf(un));
     out[0] = un;
     out[1] = fma_r(p[2], un, p[3]);
@@ -574,7 +564,7 @@ struct BatchFwd {
     o.rm.rmap = base.rm.rmap + d.rmap0;
     o.rm.rnext = base.rm.rnext + d.rnext0;
     o.rm.nrec = d.nrec;
-    o.tr = base.tr + d.tr0;
+    o.rv = base.rv ? base.rv + d.rnext0 : nullptr;
     o.nx = d.nx;
     o.ny = d.ny;
     o.rg = rings + d.ring0;
@@ -656,7 +646,7 @@ struct BatchLam {
     o.rm.rmap = base.rm.rmap + d.rmap0;
     o.rm.rnext = base.rm.rnext + d.rnext0;
     o.rm.nrec = d.nrec;
-    o.tr = base.tr + d.tr0;
+    o.gin = base.gin ? base.gin + d.rnext0 : nullptr;
     o.nx = d.nx;
     o.ny = d.ny;
     o.ring = {rings + d.ring0 + BR_U, (unsigned *)(rings + d.ring0 + BR_U + 4)};
@@ -698,7 +688,15 @@ struct BatchLam {
   case 20: return F<OP, 1, 8, 2, 2, 32>(__VA_ARGS__);        \
   case 21: return F<OP, 2, 8, 2, 2, 32>(__VA_ARGS__);        \
   case 22: return F<OP, 1, 12, 2, 2, 32>(__VA_ARGS__);       \
-  case 23: return F<OP, 2, 2, 2, 2, 32>(__VA_ARGS__);
+  case 23: return F<OP, 2, 2, 2, 2, 32>(__VA_ARGS__);        \
+  case 24: return F<OP, 1, 4, 4, 1, 16>(__VA_ARGS__);        \
+  case 25: return F<OP, 1, 2, 4, 1, 16>(__VA_ARGS__);        \
+  case 26: return F<OP, 2, 2, 4, 1, 16>(__VA_ARGS__);        \
+  case 27: return F<OP, 1, 8, 4, 1, 16>(__VA_ARGS__);        \
+  case 28: return F<OP, 1, 1, 4, 1, 8>(__VA_ARGS__);         \
+  case 29: return F<OP, 1, 3, 4, 1, 8>(__VA_ARGS__);         \
+  case 30: return F<OP, 1, 4, 4, 2, 16>(__VA_ARGS__);        \
+  case 31: return F<OP, 1, 2, 4, 2, 16>(__VA_ARGS__);
 
 
 inline Grid make_grid(const Geometry &geo, const TileShape &ts, int zc) {
@@ -707,9 +705,10 @@ inline Grid make_grid(const Geometry &geo, const TileShape &ts, int zc) {
 }
 
 template <class Op, int RY, int WY, int VX, int LA, int LX>
-hipError_t launch_shape(const Geometry &geo, int zc, const Op &op, hipStream_t st) {
-  if (VX == 2 && geo.nx % 2) return hipErrorInvalidValue;
-  const Grid g = make_grid(geo, {RY, WY, VX, LA, LX}, zc);
+hipError_t launch_shape(const Geometry &geo, const Tune &tu, const Op &op, hipStream_t st) {
+  if (geo.nx % VX) return hipErrorInvalidValue;
+  Grid g = make_grid(geo, {RY, WY, VX, LA, LX}, tu.zchunk);
+  g.back = tu.back;
   const int nb = g.ntx * g.nty * g.ntz;
   hipLaunchKernelGGL((march_kernel<Op, RY, WY, VX, LA, LX>), dim3(nb), dim3(kTX * WY), 0, st,
                      g, geo.taps, geo.sponge, op);
@@ -719,7 +718,7 @@ hipError_t launch_shape(const Geometry &geo, int zc, const Op &op, hipStream_t s
 template <class Op>
 hipError_t launch(const Geometry &geo, const Tune &tu, const Op &op, hipStream_t st) {
   switch (tu.shape) {
-    BORN_SHAPE_CASES(launch_shape, Op, geo, tu.zchunk, op, st)
+    BORN_SHAPE_CASES(launch_shape, Op, geo, tu, op, st)
     default: return hipErrorInvalidValue;
   }
 }
@@ -733,16 +732,17 @@ T *as(const void *p) {
 }
 
 template <class BOp, int RY, int WY, int VX, int LA, int LX>
-hipError_t launch_batch_shape(const Taps &taps, int zc, const BatchCommon &b,
-                                     const BOp &op, hipStream_t st) {
+hipError_t launch_batch_shape(const Taps &taps, const Tune &tu, const BatchCommon &b,
+                              const BOp &op, hipStream_t st) {
   if (b.nshots < 1 || b.nshots > kMaxBatch) return hipErrorInvalidValue;
   BatchTiles bt{};
   bt.n = b.nshots;
-  bt.zc = zc > 0 ? zc : 32;
+  bt.zc = tu.zchunk > 0 ? tu.zchunk : 32;
+  bt.back = tu.back;
   int tiles = 0;
   for (int s = 0; s < b.nshots; s++) {
     const ShotDesc &d = b.host_desc[s];
-    if (VX == 2 && d.nx % 2) return hipErrorInvalidValue;
+    if (d.nx % VX) return hipErrorInvalidValue;
     const Grid g = tile_grid(d.nx, d.ny, d.nz, LX * VX, RY * (kTX * WY / LX), bt.zc);
     bt.tile0[s] = tiles;
     tiles += g.ntx * g.nty * g.ntz;
@@ -757,7 +757,7 @@ template <class BOp>
 hipError_t launch_batch(const Taps &taps, const Tune &tu, const BatchCommon &b,
                                const BOp &op, hipStream_t st) {
   switch (tu.shape) {
-    BORN_SHAPE_CASES(launch_batch_shape, BOp, taps, tu.zchunk, b, op, st)
+    BORN_SHAPE_CASES(launch_batch_shape, BOp, taps, tu, b, op, st)
     default: return hipErrorInvalidValue;
   }
 }
@@ -776,8 +776,7 @@ hipError_t fwd_step(const Geometry &geo, const Tune &tu, const FwdStep &a, hipSt
   op.vel = a.vel; op.model = a.model; op.vm = (const float2 *)a.vm; op.hist = as<T>(a.hist);
   if (!a.vm) return hipErrorInvalidValue;
   op.pts = to_points(a.src); op.amp = a.amp;
-  op.rm = a.rec; op.tr = a.tr; op.tab = a.tab; op.id = a.id;
-  op.extract = a.extract; op.nx = geo.nx; op.ny = geo.ny;
+  op.rm = a.rec; op.rv = a.rv; op.nx = geo.nx; op.ny = geo.ny;
   op.rg = a.rg; op.slots = pack_slots(a.h.sl);
   op.gain = a.h.gain; op.tapsum = a.h.tapsum; op.hscale = a.hscale;
   op.nlev = (uint32_t)geo.nx * geo.ny * geo.nz;
@@ -800,8 +799,7 @@ template <class T>
 hipError_t lam_step(const Geometry &geo, const Tune &tu, const LamStep &a, hipStream_t st) {
   LamOp<T> op{};
   op.u1 = as<T>(a.u1); op.u0 = as<T>(a.u0); op.vel = a.vel; op.sig = as<T>(a.sig);
-  op.acc = a.acc; op.rm = a.rec; op.tr = a.tr; op.tab = a.tab; op.id = a.id;
-  op.inject = a.inject; op.nx = geo.nx; op.ny = geo.ny;
+  op.acc = a.acc; op.rm = a.rec; op.gin = a.gin; op.nx = geo.nx; op.ny = geo.ny;
   op.ring = a.ring; op.sl = a.h.sl; op.gain = a.h.gain; op.inj = a.inj;
   op.trmax = a.trmax; op.hscale = a.hscale;
   op.nlev = (uint32_t)geo.nx * geo.ny * geo.nz;
@@ -820,8 +818,7 @@ hipError_t batch_fwd_step(const Taps &taps, const Tune &tu, const BatchFwdStep &
   op.srn = (PairOf<T> *)a.s0;
   op.vel = a.vel; op.model = a.model; op.hist = nullptr;
   op.pts = to_points(a.src); op.amp = a.amp;
-  op.rm = a.rec; op.tr = a.tr; op.tab = a.tab; op.id = a.id;
-  op.extract = a.extract;
+  op.rm = a.rec; op.rv = a.rv;
   op.slots = pack_slots(a.h.sl); op.tapsum = a.h.tapsum; op.hscale = nullptr;
   bop.sponge = b.sponge; bop.rings = b.rings; bop.desc = b.desc; bop.step = b.step;
   bop.npts_total = b.npts_total;
@@ -850,8 +847,7 @@ hipError_t batch_lam_step(const Taps &taps, const Tune &tu, const BatchLamStep &
   BatchLam<T> bop{};
   auto &op = bop.base;
   op.u1 = as<T>(a.u1); op.u0 = as<T>(a.u0); op.vel = a.vel; op.sig = as<T>(a.sig);
-  op.acc = a.acc; op.rm = a.rec; op.tr = a.tr; op.tab = a.tab; op.id = a.id;
-  op.inject = a.inject; op.sl = a.h.sl; op.inj = a.inj; op.hscale = a.hscale;
+  op.acc = a.acc; op.rm = a.rec; op.gin = a.gin; op.sl = a.h.sl; op.inj = a.inj; op.hscale = a.hscale;
   bop.sponge = b.sponge; bop.rings = b.rings; bop.desc = b.desc; bop.step = b.step;
   bop.npts_total = b.npts_total;
   return launch_batch(taps, tu, b, bop, st);
