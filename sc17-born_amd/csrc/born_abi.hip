@@ -343,46 +343,36 @@ born::Tune sweep(born::Tune t, int k) {
   return t;
 }
 
-// Autotuner: time every tile shape x z chunk for one step kernel and keep
-// the fastest in *tune / *tune_ms (ms per launch; the four fastest of a
-// first pass are timed again, round-robin, over more launches).  run(tune) must launch the kernel on
-// scratch buffers only.  Pair shapes (2 cells per lane) need even_nx.
+// Autotuner: search tile shape x z chunk for one step kernel and keep the
+// fastest in *tune / *tune_ms (ms per launch).  run(tune) must launch the
+// kernel on scratch buffers only, tiles(shape) is its number of xy tiles (of
+// every shot of a batch), nzi its interior planes (the most of a batch's
+// shots).  xdiv: cells per lane must divide it.
 //
-// z chunks: 32, 64 and 128 planes and, for nzi > 0 interior planes, every
-// length that splits nzi evenly into k = 1..16 chunks (ceil(nzi / k), at
-// least 16 planes), so that no block marches more planes than the others
-// (at 296 planes, chunks of 60 end with one of 56 where chunks of 64 end
-// with one of 40) and the number of blocks can match what the CUs hold at
-// once.
-constexpr int kMaxZChunks = 19;
-static int zchunk_candidates(int nzi, int (&zcs)[kMaxZChunks]) {
-  int n = 0;
-  auto add = [&](int zc) {
-    for (int i = 0; i < n; i++)
-      if (zcs[i] == zc) return;
-    if (n < kMaxZChunks) zcs[n++] = zc;
-  };
-  for (int target : {32, 64, 128}) add(target);
-  if (nzi > 0)
-    for (int k = 1; k <= 16; k++) {
-      const int zc = (nzi + k - 1) / k;
-      if (zc >= 16) add(zc);
-    }
-  return n;
-}
-
-template <class F>
-int autotune_into(born_ctx *ctx, born::Tune *tune, float *tune_ms, int xdiv, int nzi,
+// z chunks split nzi evenly (ceil(nzi / k) for k chunks, two planes or more):
+// no block marches more planes than the others, and the number of blocks can
+// match what the CUs hold at once.  Which k is best depends on the tile and
+// the grid: a launch wants some hundreds of blocks at least (with 64^3 cells,
+// chunks of 2 planes: 7.4 us per FP32 forward step; of 19 planes, 23.6 us) and
+// few planes read twice (304^3: chunks of 74 planes, 164 us; of 37, 172 us).
+// So each shape (with one plane of lookahead) is first timed with the chunks
+// that come nearest to five numbers of blocks, then the best five shapes with
+// every chunk that gives from half to twice as many blocks as their best, and
+// with two planes of lookahead; the four fastest of all are timed again,
+// round-robin.  The search takes 0.5 s of a 304^3 FP32 pair's first pass,
+// where a grid of every shape and 16 chunk lengths took 1.2 s.
+constexpr int kMinBlocks = 128, kMaxBlocks = 5120;
+template <class F, class B>
+int autotune_into(born_ctx *ctx, born::Tune *tune, float *tune_ms, int xdiv, int nzi, B tiles,
                   F run) {
   if (!ctx->autotune || *tune_ms >= 0.f) return BORN_OK;
-  int zcs[kMaxZChunks];
-  const int nzc = zchunk_candidates(nzi, zcs);
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
-  // ms per launch of `reps` launches after one untimed launch
+  // ms per launch of `reps` launches, after an untimed one if there are more
+  // than one
   auto time = [&](const born::Tune &t, int reps, float *ms) -> int {
-    HIPCHK(run(sweep(t, 1)));
+    if (reps > 1) HIPCHK(run(sweep(t, 1)));
     HIPCHK(hipEventRecord(e0, ctx->stream));
     for (int r = 0; r < reps; r++) HIPCHK(run(sweep(t, r)));
     HIPCHK(hipEventRecord(e1, ctx->stream));
@@ -391,27 +381,89 @@ int autotune_into(born_ctx *ctx, born::Tune *tune, float *tune_ms, int xdiv, int
     *ms /= reps;
     return BORN_OK;
   };
-  // every candidate over 3 launches
-  std::vector<std::pair<float, born::Tune>> cand;
-  for (int sh = 0; sh < born::kNumShapes; sh++)
-    for (int zi = 0; zi < nzc; zi++) {
-      if (xdiv % born::kShapes[sh].vx) continue;
-      const born::Tune t{sh, ctx->zchunk > 0 ? ctx->zchunk : zcs[zi]};
-      if (ctx->zchunk > 0 && zi > 0) continue;
-      float ms = 0.f;
-      CHK(time(t, 3, &ms));
-      cand.push_back({ms, t});
+  struct Cand {
+    float ms;
+    born::Tune t;
+  };
+  std::vector<Cand> cand;
+  float fastest = 1e30f;
+  auto try_one = [&](int sh, int zc) -> int {
+    for (const Cand &c : cand)
+      if (c.t.shape == sh && c.t.zchunk == zc) return BORN_OK;
+    Cand c{0.f, {sh, zc}};
+    // one launch tells the hopeless ones; launches of a few us are timed over
+    // more of them
+    CHK(time(c.t, 1, &c.ms));
+    if (c.ms < 1.5f * fastest) CHK(time(c.t, c.ms < .03f ? 10 : 3, &c.ms));
+    fastest = std::min(fastest, c.ms);
+    cand.push_back(c);
+    return BORN_OK;
+  };
+  auto faster = [](const Cand &a, const Cand &b) { return a.ms < b.ms; };
+  // the z chunks of a shape with lo to hi blocks, coarse to fine; if none,
+  // the one nearest to that
+  auto chunks = [&](int sh, double lo, double hi) {
+    std::vector<int> zcs;
+    const int n = std::max(1, tiles(sh)), kmax = std::max(1, nzi / 2);
+    int near = 1;
+    for (int k = 1; k <= kmax; k++) {
+      if ((double)n * k < lo) near = k;
+      if ((double)n * k < lo || (double)n * k > hi) continue;
+      const int zc = (nzi + k - 1) / k;
+      if (zcs.empty() || zcs.back() != zc) zcs.push_back(zc);
     }
-  std::sort(cand.begin(), cand.end(),
-            [](const auto &a, const auto &b) { return a.first < b.first; });
-  // the four fastest again, round-robin over three rounds of 30 launches
-  // (a drift of the clocks during the search then favours none of them)
+    if (zcs.empty()) zcs.push_back((nzi + near - 1) / near);
+    return zcs;
+  };
+  for (int sh = 0; sh < born::kNumShapes; sh++) {
+    if (xdiv % born::kShapes[sh].vx || born::kShapes[sh].la != 1) continue;
+    if (ctx->zchunk > 0) {
+      CHK(try_one(sh, ctx->zchunk));
+      continue;
+    }
+    const std::vector<int> zcs = chunks(sh, kMinBlocks, kMaxBlocks);
+    const int n = std::max(1, tiles(sh));
+    for (double target : {256., 512., 768., 1280., 2300.}) {
+      int best = zcs[0];
+      double off = 1e30;
+      for (int zc : zcs) {
+        const double nb = (double)n * ((nzi + zc - 1) / zc);
+        const double d = nb > target ? nb / target : target / nb;
+        if (d < off) {
+          off = d;
+          best = zc;
+        }
+      }
+      CHK(try_one(sh, best));
+    }
+  }
+  std::vector<Cand> order = cand;
+  std::sort(order.begin(), order.end(), faster);
+  std::vector<int> done;
+  for (size_t i = 0; i < order.size() && done.size() < 5; i++) {
+    const int sh = order[i].t.shape, zc = order[i].t.zchunk;
+    if (std::find(done.begin(), done.end(), sh) != done.end()) continue;
+    done.push_back(sh);
+    const born::TileShape &ts = born::kShapes[sh];
+    for (int l = 0; l < born::kNumShapes; l++) {
+      const born::TileShape &o = born::kShapes[l];
+      if (o.la == 2 && o.ry == ts.ry && o.wy == ts.wy && o.vx == ts.vx && o.lx == ts.lx)
+        CHK(try_one(l, zc));
+    }
+    if (ctx->zchunk > 0) continue;
+    const double nb = (double)std::max(1, tiles(sh)) * ((nzi + zc - 1) / zc);
+    for (int z : chunks(sh, nb / 2, nb * 2)) CHK(try_one(sh, z));
+  }
+  std::sort(cand.begin(), cand.end(), faster);
+  // the four fastest again, round-robin over three rounds of about 2 ms, 8 to
+  // 30 launches (a drift of the clocks during the search then favours none)
   const size_t top = std::min<size_t>(cand.size(), 4);
+  const int reps = (int)std::min(30.f, std::max(8.f, 2.f / std::max(cand[0].ms, 1e-3f)));
   float sum[4] = {0.f, 0.f, 0.f, 0.f};
   for (int round = 0; round < 3; round++)
     for (size_t i = 0; i < top; i++) {
       float ms = 0.f;
-      CHK(time(cand[i].second, 30, &ms));
+      CHK(time(cand[i].t, reps, &ms));
       sum[i] += ms / 3.f;
     }
   float best = 1e30f;
@@ -419,7 +471,7 @@ int autotune_into(born_ctx *ctx, born::Tune *tune, float *tune_ms, int xdiv, int
   for (size_t i = 0; i < top; i++)
     if (sum[i] < best) {
       best = sum[i];
-      bt = cand[i].second;
+      bt = cand[i].t;
     }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
@@ -430,8 +482,9 @@ int autotune_into(born_ctx *ctx, born::Tune *tune, float *tune_ms, int xdiv, int
 
 template <class F>
 int autotune(born_ctx *ctx, int kind, F run) {
-  return autotune_into(ctx, &ctx->tune[kind], &ctx->tune_ms[kind], x_div(ctx->nx),
-                       ctx->nz - 2 * born::kH, run);
+  return autotune_into(
+      ctx, &ctx->tune[kind], &ctx->tune_ms[kind], x_div(ctx->nx), ctx->nz - 2 * born::kH,
+      [&](int sh) { return tile_count(ctx->nx, ctx->ny, sh); }, run);
 }
 
 // The same for a two-step kernel: its shapes and z chunks that split the
@@ -2622,7 +2675,8 @@ int born_batch_forward(born_batch *b, int jt, int nt, int scatter) {
     HIPCHK(born::launch_batch_ring_init(b->d_rings, b->nshots, ctx->stream));
     born::BatchFwdStep t = batch_step(b, 0, jt, scatter, storage, 0);
     t.a.rv = nullptr;
-    CHK(autotune_into(ctx, &b->tune[kind], &b->tune_ms[kind], b->xdiv, 0,
+    CHK(autotune_into(ctx, &b->tune[kind], &b->tune_ms[kind], b->xdiv, b->max_nzi,
+                      [&](int sh) { return batch_tiles(b, sh); },
                       [&](const born::Tune &tu) {
                         return born::launch_batch_fwd_step(taps, tu, t, ctx->stream);
                       }));
@@ -2781,7 +2835,8 @@ int born_batch_adjoint_exact(born_batch *b, int jt, int nt, int scatter) {
     t.a.s1 = s_cur; t.a.s0 = s_old; t.a.vel = b->d_vel; t.a.sig = b->d_acc;
     t.a.src = {b->d_pts, 0}; t.a.amp = b->d_amp; t.a.scatter = scatter;
     t.a.h = hstate(0); t.a.hscale = b->d_hscale;
-    CHK(autotune_into(ctx, &b->tune[skind], &b->tune_ms[skind], b->xdiv, 0,
+    CHK(autotune_into(ctx, &b->tune[skind], &b->tune_ms[skind], b->xdiv, b->max_nzi,
+                      [&](int sh) { return batch_tiles(b, sh); },
                       [&](const born::Tune &tu) {
                         return born::launch_batch_srec_step(taps, tu, t, ctx->stream);
                       }));
@@ -2791,7 +2846,8 @@ int born_batch_adjoint_exact(born_batch *b, int jt, int nt, int scatter) {
     l.a.rec.plane_slot = b->d_slot; l.a.rec.rmap = b->d_rmap; l.a.rec.rnext = b->d_rnext;
     l.a.rec.ntb = b->ntb; l.a.rec.shared = b->rec_shared;
     l.a.h = hstate(0); l.a.inj = ctx->tabd_abs; l.a.hscale = b->d_hscale;
-    CHK(autotune_into(ctx, &b->tune[lkind], &b->tune_ms[lkind], b->xdiv, 0,
+    CHK(autotune_into(ctx, &b->tune[lkind], &b->tune_ms[lkind], b->xdiv, b->max_nzi,
+                      [&](int sh) { return batch_tiles(b, sh); },
                       [&](const born::Tune &tu) {
                         return born::launch_batch_lam_step(taps, tu, l, ctx->stream);
                       }));
