@@ -124,9 +124,8 @@ __device__ __forceinline__ const T &at(const T *p, uint32_t o) {
 // A vector memory instruction that reads a scalar register written by a
 // vector instruction (v_readlane, as in a reload of a spilled scalar) needs
 // 5 wait states before it, which the compiler does not insert for inline
-// asm: each store starts with s_nop 4.  NT adds the non-temporal hint: no
-// step reads a new level back before the next launch, and the hint took 6 %
-// off the FP32 forward step at 304^3.
+// asm: each store starts with s_nop 4.  NT adds the non-temporal hint (where
+// it pays is measured at the ops).
 template <bool NT>
 __device__ __forceinline__ void st_b8(void *p, uint32_t off, unsigned char v) {
   if constexpr (NT)
@@ -639,16 +638,16 @@ __device__ __forceinline__ void ld_stream(const __half *p, uint32_t po, uint32_t
                                           float (&v)[VX], uint32_t = 0) {
   ld_vec<VX>(p, po, o, inv, v);
 }
-// two FP32 fields interleaved cell by cell (non-temporal)
+// two FP32 fields interleaved cell by cell
 template <int VX>
-__device__ __forceinline__ void ld_stream2(const float2 *p, uint32_t po, uint32_t o,
+__device__ __forceinline__ void ld_vec2(const float2 *p, uint32_t po, uint32_t o,
                                            float (&a)[VX], float (&b)[VX]) {
   const char *q = adv(p, (uint64_t)po * 8u);
 #pragma unroll
   for (int h = 0; h < (VX + 1) / 2; h++) {
     constexpr int N = VX == 1 ? 2 : 4;
     uint32_t u[N];
-    ld_words<uint32_t, N, true>(q + 16 * h, o * 8u, u);
+    ld_words<uint32_t, N>(q + 16 * h, o * 8u, u);
 #pragma unroll
     for (int i = 0; i < N / 2; i++) {
       a[2 * h + i] = __uint_as_float(u[2 * i]);

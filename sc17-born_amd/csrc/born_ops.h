@@ -74,8 +74,15 @@ __device__ __forceinline__ float amp_sum(const Points &pts, const float *amp) {
 }
 
 // ---------------------------------------------------------------- forward
-// NT: non-temporal hint on the stores and FP32 pointwise loads (the shot
-// batch runs without it, see BatchFwd)
+// NT: the single-shot forward: non-temporal hint on the FP32 and 24-bit
+// stores, velocity and model as one stream (the shot batch: see BatchFwd).
+// The loads take no hint: what a step reads the next one reads or overwrites,
+// and a load with the hint leaves nothing in the 256 MB memory-side cache.
+// FP32, us per step with the hint on the pointwise loads -> without: 160^3
+// 31.6 -> 26.4 (dV scatter 35.5 -> 26.1), 224^3 73.7 -> 63.9 (83.7 -> 61.7),
+// 304^3 175.1 -> 172.6 (207.6 -> 194.1).  The stores keep it in FP32: 304^3
+// 172.4 with, 177.9 without.  FP16 without any: 160^3 38.1 -> 36.1, 224^3 72.8
+// -> 66.9, 304^3 127.9 -> 128.9.
 template <int SCATTER, class T, bool NT = true>
 struct FwdOp {
   static constexpr bool H = kScaled<T>;
@@ -178,15 +185,12 @@ struct FwdOp {
         p[0][v] = sr[0][v];
         p[1][v] = sr[1][v];
       }
-    } else if constexpr (NT) {
-      ld_stream<VX>(s0, po, o, b.io[0], p[0], nlev);
-      ld_stream<VX>(r0, po, o, b.io[1], p[1], nlev);
     } else {
       ld_vec<VX>(s0, po, o, b.io[0], p[0], nlev);
       ld_vec<VX>(r0, po, o, b.io[1], p[1], nlev);
     }
     if constexpr (NT) {
-      ld_stream2<VX>(vm, po, o, p[2], p[3]);
+      ld_vec2<VX>(vm, po, o, p[2], p[3]);
     } else {
       ld_vec<VX>(vel, po, o, 1.f, p[2]);
       ld_vec<VX>(model, po, o, 1.f, p[3]);
@@ -196,7 +200,7 @@ struct FwdOp {
   __device__ void storev(const Blk2 &b, uint32_t po, uint32_t o,
                          const float (&out)[NOUT][VX]) const {
     if constexpr (PAIRED) {
-      st_pair<VX, NT>(srn, po, o, out[0], out[1], b.sn, nlev);
+      st_pair<VX, NT && kSplit<T>>(srn, po, o, out[0], out[1], b.sn, nlev);
     } else {
       st_vec<VX, NT>(s_new, po, o, out[0], b.sn[0], nlev);
       st_vec<VX, NT>(r0, po, o, out[1], b.sn[1], nlev);
@@ -320,9 +324,11 @@ struct RadjOp {
   template <int VX>
   __device__ void storev(uint32_t, uint32_t po, uint32_t o,
                          const float (&out)[NOUT][VX]) const {
-    if (s_prop) st_vec<VX>(s0, po, o, out[0], 1.f);
-    st_vec<VX>(r0, po, o, out[1], 1.f);
-    st_vec<VX>(img, po, o, out[2], 1.f);
+    // no hint: every array here is read again by the next step (304^3 227.9 ->
+    // 223.4 us, 160^3 29.4 -> 27.9; with the hint on the loads too, 160^3 35)
+    if (s_prop) st_vec<VX, false>(s0, po, o, out[0], 1.f);
+    st_vec<VX, false>(r0, po, o, out[1], 1.f);
+    st_vec<VX, false>(img, po, o, out[2], 1.f);
   }
   __device__ void cell(uint32_t, const SrcPln &pl, const CellArgs &c, const float *lap,
                        const float *ctr, const float *p, float (&out)[NOUT],
