@@ -515,7 +515,7 @@ __device__ __forceinline__ void split_two(uint32_t h, uint32_t l, float &a, floa
 }
 
 // (n a multiple of VX: the lo bytes of VX cells are aligned to VX bytes)
-template <int VX>
+template <int VX, bool = false>
 __device__ __forceinline__ void ld_vec(const Split *p, uint32_t po, uint32_t o, float,
                                        float (&v)[VX], uint32_t n) {
   const char *bh = adv(p, (uint64_t)po * 2u), *bl = adv(p, (uint64_t)n * 2u + po);
@@ -528,11 +528,6 @@ __device__ __forceinline__ void ld_vec(const Split *p, uint32_t po, uint32_t o, 
     split_two(h[0], l, v[0], v[1]);
     if constexpr (VX == 4) split_two(h[1], l >> 16, v[2], v[3]);
   }
-}
-template <int VX>
-__device__ __forceinline__ void ld_stream(const Split *p, uint32_t po, uint32_t o, float inv,
-                                          float (&v)[VX], uint32_t n) {
-  ld_vec<VX>(p, po, o, inv, v, n);
 }
 template <int VX, bool NT = true>
 __device__ __forceinline__ void st_vec(Split *p, uint32_t po, uint32_t o,
@@ -599,7 +594,7 @@ __device__ __forceinline__ void st_pair(SplitPair *p, uint32_t po, uint32_t o,
   }
 }
 
-// ---- one field per array, FP32 or FP16
+// ---- one field per array, FP32 (NT: with the non-temporal hint) or FP16
 template <int VX, bool NT = false>
 __device__ __forceinline__ void ld_vec(const float *p, uint32_t po, uint32_t o, float,
                                        float (&v)[VX], uint32_t = 0) {
@@ -608,7 +603,7 @@ __device__ __forceinline__ void ld_vec(const float *p, uint32_t po, uint32_t o, 
 #pragma unroll
   for (int i = 0; i < VX; i++) v[i] = __uint_as_float(u[i]);
 }
-template <int VX>
+template <int VX, bool = false>
 __device__ __forceinline__ void ld_vec(const __half *p, uint32_t po, uint32_t o, float inv,
                                        float (&v)[VX], uint32_t = 0) {
   const char *b = adv(p, (uint64_t)po * 2u);
@@ -623,20 +618,6 @@ __device__ __forceinline__ void ld_vec(const __half *p, uint32_t po, uint32_t o,
       v[2 * i + 1] = __high2float(as_half2(u[i])) * inv;
     }
   }
-}
-// The same loads with the non-temporal hint, for inputs a launch reads once
-// (the pointwise operands of a cell).
-template <int VX>
-__device__ __forceinline__ void ld_stream(const float *p, uint32_t po, uint32_t o, float inv,
-                                          float (&v)[VX], uint32_t = 0) {
-  ld_vec<VX, true>(p, po, o, inv, v);
-}
-// FP16 levels keep the plain loads: with the hint the FP16 adjoint-state
-// and background steps ran 15-20 % slower (304^3, 2- and 4-byte lanes).
-template <int VX>
-__device__ __forceinline__ void ld_stream(const __half *p, uint32_t po, uint32_t o, float inv,
-                                          float (&v)[VX], uint32_t = 0) {
-  ld_vec<VX>(p, po, o, inv, v);
 }
 // two FP32 fields interleaved cell by cell
 template <int VX>

@@ -175,7 +175,8 @@ __global__ void transpose_kernel(float *dst, const float *src, int n0, int n1) {
       {1, 8, 2, LA, 32}, {2, 8, 2, LA, 32}, {1, 12, 2, LA, 32}, {2, 2, 2, LA, 32}
 const TileShape kShapes[kNumShapes] = {
     BORN_TILES(1),    BORN_TILES(2),    {1, 4, 4, 1, 16}, {1, 2, 4, 1, 16}, {2, 2, 4, 1, 16},
-    {1, 8, 4, 1, 16}, {1, 1, 4, 1, 8},  {1, 3, 4, 1, 8},  {1, 4, 4, 2, 16}, {1, 2, 4, 2, 16}};
+    {1, 8, 4, 1, 16}, {1, 1, 4, 1, 8},  {1, 3, 4, 1, 8},  {1, 4, 4, 2, 16}, {1, 2, 4, 2, 16},
+    {1, 2, 2, 1, 16}, {2, 1, 2, 1, 16}};
 #undef BORN_TILES
 
 // the launchers of born_launch.h: dispatch on storage and scatter to the

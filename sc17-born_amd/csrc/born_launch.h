@@ -22,7 +22,7 @@ struct Geometry {
 struct TileShape {
   int ry, wy, vx, la, lx;
 };
-constexpr int kNumShapes = 32;
+constexpr int kNumShapes = 34;
 extern const TileShape kShapes[kNumShapes];
 
 // Launch configuration of one step kernel: tile shape, z planes per block and

@@ -200,7 +200,7 @@ struct FwdOp {
   __device__ void storev(const Blk2 &b, uint32_t po, uint32_t o,
                          const float (&out)[NOUT][VX]) const {
     if constexpr (PAIRED) {
-      st_pair<VX, NT && kSplit<T>>(srn, po, o, out[0], out[1], b.sn, nlev);
+      st_pair<VX, false>(srn, po, o, out[0], out[1], b.sn, nlev);
     } else {
       st_vec<VX, NT>(s_new, po, o, out[0], b.sn[0], nlev);
       st_vec<VX, NT>(r0, po, o, out[1], b.sn[1], nlev);
@@ -411,18 +411,17 @@ struct SrecOp {
   template <int VX>
   __device__ void prefetchv(const Blk1 &b, float (&p)[NPRE][VX], uint32_t po,
                             uint32_t o) const {
-    ld_stream<VX>(s0, po, o, b.io, p[0], nlev);
-    // FP32: the velocity without the hint (114 -> 103 us per step at 304^3)
-    if constexpr (kNarrow<T>)
-      ld_stream<VX>(vel, po, o, 1.f, p[1]);
-    else
-      ld_vec<VX>(vel, po, o, 1.f, p[1]);
+    // FP32: the old level and the stores with the non-temporal hint; narrow
+    // levels without any (FP16 background and adjoint state, us per step of
+    // each together: 304^3 196.9 -> 184.9, 160^3 49.7 -> 47.1)
+    ld_vec<VX, !kNarrow<T>>(s0, po, o, b.io, p[0], nlev);
+    ld_vec<VX>(vel, po, o, 1.f, p[1]);
   }
   template <int VX>
   __device__ void storev(const Blk1 &b, uint32_t po, uint32_t o,
                          const float (&out)[NOUT][VX]) const {
-    st_vec<VX>(s_new, po, o, out[0], b.sn, nlev);
-    if (sig) st_vec<VX>(sig, po, o, out[1], b.sh, nlev);
+    st_vec<VX, !kNarrow<T>>(s_new, po, o, out[0], b.sn, nlev);
+    if (sig) st_vec<VX, !kNarrow<T>>(sig, po, o, out[1], b.sh, nlev);
   }
   __device__ void cell(const Blk1 &, uint32_t pm, const CellArgs &c, const float *lap,
                        const float *ctr, const float *p, float (&out)[NOUT],
@@ -494,24 +493,19 @@ struct LamOp {
   template <int VX>
   __device__ void prefetchv(const Blk1 &b, float (&p)[NPRE][VX], uint32_t po,
                             uint32_t o) const {
-    ld_stream<VX>(u0, po, o, b.io, p[0], nlev);
-    ld_stream<VX>(sig, po, o, b.sh, p[2], nlev);
-    // FP32: velocity and image without the non-temporal hint (read, and the
-    // image written, every step: 143 against 155 us per step at 304^3);
-    // the FP16 step is faster with it
-    if constexpr (kNarrow<T>) {
-      ld_stream<VX>(vel, po, o, 1.f, p[1]);
-      ld_stream<VX>(acc, po, o, 1.f, p[3]);
-    } else {
-      ld_vec<VX>(vel, po, o, 1.f, p[1]);
-      ld_vec<VX>(acc, po, o, 1.f, p[3]);
-    }
+    // FP32: the non-temporal hint on the levels, not on velocity and image
+    // (304^3 134.8 us; without any 143.5); narrow levels without any (24-bit
+    // 224^3 61.7 -> 58.4)
+    ld_vec<VX, !kNarrow<T>>(u0, po, o, b.io, p[0], nlev);
+    ld_vec<VX, !kNarrow<T>>(sig, po, o, b.sh, p[2], nlev);
+    ld_vec<VX>(vel, po, o, 1.f, p[1]);
+    ld_vec<VX>(acc, po, o, 1.f, p[3]);
   }
   template <int VX>
   __device__ void storev(const Blk1 &b, uint32_t po, uint32_t o,
                          const float (&out)[NOUT][VX]) const {
-    st_vec<VX>(u0, po, o, out[0], b.sn, nlev);
-    st_vec<VX, kNarrow<T>>(acc, po, o, out[1], 1.f);
+    st_vec<VX, !kNarrow<T>>(u0, po, o, out[0], b.sn, nlev);
+    st_vec<VX, false>(acc, po, o, out[1], 1.f);
   }
   __device__ void cell(const Blk1 &, int slot, const CellArgs &c, const float *lap,
                        const float *ctr, const float *p, float (&out)[NOUT],
@@ -702,7 +696,9 @@ struct BatchLam {
   case 28: return F<OP, 1, 1, 4, 1, 8>(__VA_ARGS__);         \
   case 29: return F<OP, 1, 3, 4, 1, 8>(__VA_ARGS__);         \
   case 30: return F<OP, 1, 4, 4, 2, 16>(__VA_ARGS__);        \
-  case 31: return F<OP, 1, 2, 4, 2, 16>(__VA_ARGS__);
+  case 31: return F<OP, 1, 2, 4, 2, 16>(__VA_ARGS__);        \
+  case 32: return F<OP, 1, 2, 2, 1, 16>(__VA_ARGS__);        \
+  case 33: return F<OP, 2, 1, 2, 1, 16>(__VA_ARGS__);
 
 
 inline Grid make_grid(const Geometry &geo, const TileShape &ts, int zc) {
