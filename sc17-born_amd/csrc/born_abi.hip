@@ -47,6 +47,7 @@ struct born_ctx {
   int autotune = 1;
   born::Tune tune[24];
   float tune_ms[24];
+  bool tuned_sr[24] = {};  // the kernel ran last with s and r together (tuned_slot)
   int pairs = 0;  // two-step forward launches for FP32 levels: 0 off, 1 auto, 2 on
 
   int nsinc_s = 0, jts = 0, nsinc_d = 0, jtd = 0;
@@ -82,6 +83,8 @@ struct born_ctx {
   float *d_ckring = nullptr;  // ring snapshot per checkpoint (8 words each)
   size_t ckring_cap = 0;
 
+  // four levels, one allocation (d_w[0]): a level of s and r together takes
+  // d_w[0] and d_w[1], or d_w[2] and d_w[3]
   float *d_w[4] = {nullptr, nullptr, nullptr, nullptr};
   size_t w_cap = 0;  // floats per work buffer
   float *d_w2[4] = {nullptr, nullptr, nullptr, nullptr};  // levels k+1, k+2 of pairs
@@ -261,9 +264,16 @@ born::RecWindow rec_steps(const born_ctx *c, int it0, int n, int jt) {
 enum Kind {
   K_FWD0, K_FWD1, K_SRC, K_RADJ, K_SREC0, K_SREC1, K_LAM,
   K_FWD0H, K_FWD1H, K_SREC0H, K_SREC1H, K_LAMH, K_FWD0P, K_FWD1P, K_LAMP,
-  K_FWD0S, K_FWD1S, K_SREC0S, K_SREC1S, K_LAMS, K_NUM
+  K_FWD0S, K_FWD1S, K_SREC0S, K_SREC1S, K_LAMS, K_NUM,
+  // FP32 levels of s and r together: not numbered at the ABI, where they are
+  // part of K_FWD0, K_FWD1 and K_RADJ (see sr_kind)
+  K_FWD0SR = K_NUM, K_FWD1SR, K_RADJSR, K_SLOTS
 };
-static_assert(K_NUM <= 24, "tuning slots");
+static_assert(K_SLOTS <= 24, "tuning slots");
+// the slot of an FP32 kernel's form with s and r together (-1: it has none)
+int sr_kind(int kind) {
+  return kind == K_FWD0 ? K_FWD0SR : kind == K_FWD1 ? K_FWD1SR : kind == K_RADJ ? K_RADJSR : -1;
+}
 // the step kernels of a storage form (BORN_STORAGE_*)
 int fwd_kind(int storage, int scatter) {
   static const int k[3][2] = {{K_FWD0, K_FWD1}, {K_FWD0H, K_FWD1H}, {K_FWD0S, K_FWD1S}};
@@ -296,7 +306,7 @@ born::Tune default_tune(int tiles, int nzi) {
 }
 
 void reset_tuning(born_ctx *c) {
-  for (int k = 0; k < K_NUM; k++) {
+  for (int k = 0; k < K_SLOTS; k++) {
     // pairs: 56x16 tiles, 128 planes
     c->tune[k] = is_pair(k) ? born::Tune{0, 128}
                             : default_tune(c->nx > 0 ? tile_count(c->nx, c->ny, 0) : 768,
@@ -332,6 +342,11 @@ born::Tune tuning(const born_ctx *c, int kind) {
   born::Tune t = c->tune[kind];
   if (c->zchunk > 0) t.zchunk = c->zchunk;
   return fit_nx(t, x_div(c->nx));
+}
+
+// The slot that a kernel numbered at the ABI ran with last.
+int tuned_slot(const born_ctx *c, int kind) {
+  return sr_kind(kind) >= 0 && c->tuned_sr[kind] ? sr_kind(kind) : kind;
 }
 
 // The launch of step k of a time loop: every second step marches its z chunks
@@ -583,16 +598,19 @@ int check_dims(born_ctx *ctx, int n1, int n2, int n3) {
 }
 
 // floats per work buffer: one float level, or a 24-bit level of two fields
-// stored together (6 bytes per cell)
+// stored together (6 bytes per cell); whole 256 bytes, as the buffers are
+// parts of one allocation
+size_t whole_lines(size_t floats) { return (floats + 63) / 64 * 64; }
 size_t work_floats(const born_ctx *c) {
-  return c->storage == BORN_STORAGE_F24 ? ((size_t)c->n * 3 + 1) / 2 : (size_t)c->n;
+  return whole_lines(c->storage == BORN_STORAGE_F24 ? ((size_t)c->n * 3 + 1) / 2 : (size_t)c->n);
 }
 
 int ensure_work(born_ctx *ctx) {
   const size_t need = work_floats(ctx);
   if (ctx->w_cap < need) {
     ctx->w_cap = 0;
-    for (int i = 0; i < 4; i++) CHK(dev_alloc(ctx, &ctx->d_w[i], need));
+    CHK(dev_alloc(ctx, &ctx->d_w[0], 4 * need));
+    for (int i = 1; i < 4; i++) ctx->d_w[i] = ctx->d_w[0] + i * need;
     ctx->w_cap = need;
   }
   // the forward's interleaved velocity and model, allocated with the work
@@ -1123,7 +1141,7 @@ int born_destroy(born_ctx *ctx) {
   void *bufs[] = {ctx->d_pts,   ctx->d_bx,    ctx->d_by,    ctx->d_bz,   ctx->d_tab_s,
                   ctx->d_tab_d, ctx->d_src,   ctx->d_vel1, ctx->d_vel2,
                   ctx->d_plane_slot, ctx->d_rmap, ctx->d_rnext, ctx->d_rv, ctx->d_w[0],
-                  ctx->d_w[1],  ctx->d_w[2],  ctx->d_w[3], ctx->d_w2[0],
+                  ctx->d_w2[0],
                   ctx->d_w2[1], ctx->d_w2[2], ctx->d_w2[3], ctx->d_img,
                   ctx->d_acc,   ctx->d_p0,    ctx->d_p1,   ctx->d_tr,
                   ctx->d_tr2,   ctx->d_amp,   ctx->d_seg,  ctx->d_ckpt,
@@ -1165,7 +1183,7 @@ int born_create_space(born_ctx *ctx, float d1, float d2, float d3, float bc_a,
   if (resized) {
     // every buffer of the old cell count goes, the two-step levels included
     // (ensure_work / ensure_pair_work only allocate a missing buffer)
-    for (int i = 0; i < 4; i++) CHK(dev_alloc(ctx, &ctx->d_w[i], 0));
+    CHK(dev_alloc(ctx, &ctx->d_w[0], 0));
     ctx->w_cap = 0;
     for (int i = 0; i < 4; i++) CHK(dev_alloc(ctx, &ctx->d_w2[i], 0));
     CHK(dev_alloc(ctx, &ctx->d_img, 0));
@@ -1383,7 +1401,13 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
   ctx->ck_version = -1;
   ctx->jt_state = jt;
   const Geometry geo = geometry(ctx);
-  const int kind = fwd_kind(ctx->storage, scatter);
+  // FP32 levels of s and r together (see FwdOp), unless s levels are wanted by
+  // themselves: in the history (scatter 0), in checkpoints, in a two-step
+  // launch; a segment history's gaps hold r alone, too
+  const bool pair = !half && !try_pairs && ckS == 0 && (!hist || (scatter == 1 && !ctx->seg_gap));
+  const int fkind = fwd_kind(ctx->storage, scatter);
+  const int kind = pair ? sr_kind(fkind) : fkind;
+  if (!half) ctx->tuned_sr[fkind] = pair;
   // velocity 2 and the model as one stream (8 bytes per cell; the buffer
   // comes with the work buffers)
   HIPCHK(born::launch_interleave(ctx->d_vm, ctx->d_vel2, model, n, ctx->stream));
@@ -1392,10 +1416,10 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
     CHK(ring_reset(ctx, RING_T1));
     HIPCHK(born::launch_fill(ctx->d_ring + MAX_T, 2, 0.f, ctx->stream));
     born::FwdStep t{};
-    t.s1 = ctx->d_w[1]; t.s0 = ctx->d_w[0]; t.r1 = ctx->d_w[3]; t.r0 = ctx->d_w[2];
+    t.s1 = ctx->d_w[pair ? 2 : 1]; t.s0 = ctx->d_w[0]; t.r1 = ctx->d_w[3]; t.r0 = ctx->d_w[2];
     t.vel = ctx->d_vel2; t.model = model; t.vm = ctx->d_vm;
     t.src = no_points(); t.rec = recmap(ctx);
-    t.scatter = scatter;
+    t.scatter = scatter; t.pair = pair;
     t.h = half_state(ctx, 0);
     t.rg = ctx->d_ring + RING_T0; t.hscale = ctx->d_ring + HS_T;
     // The buffers the steps below use.  With the s levels in the kept
@@ -1535,7 +1559,7 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
       std::swap(rb[1], rb[3]);
     }
   }
-  float *s_old = sb[0], *s_cur = sb[1];
+  float *s_old = sb[0], *s_cur = pair ? ctx->d_w[2] : sb[1];
   float *r_old = rb[0], *r_cur = rb[1];
   born::FwdStep a{};
   a.vel = ctx->d_vel2;
@@ -1544,6 +1568,7 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
   a.src = points(ctx);
   a.rec = recmap(ctx);
   a.scatter = scatter;
+  a.pair = pair;
   a.rg = ctx->d_ring + RING_S;
   // With scatter 0 the scatter operand of step it is s of level it+1, so a
   // kept history holds the s levels: step it reads levels it (history it-1)
@@ -1719,24 +1744,38 @@ int born_dev_rtm_adjoint(born_ctx *ctx, int nt, float *p0, float *p1, float *img
   CHK(ensure(ctx, &ctx->d_rv, &ctx->rv_cap, (size_t)rwin * ctx->nrec));
   const long long n = ctx->n;
   const Geometry geo = geometry(ctx);
+  // s and r together (see RadjOp) in the work buffers, with a pass over s
+  // before and after the loop, which cost what 20 (304^3) to 36 (160^3) of its
+  // steps gain; under 128^3 cells the step gains nothing
+  const bool pair = n >= 1 << 21 && nt >= 48;
+  const int kind = pair ? K_RADJSR : K_RADJ;
+  ctx->tuned_sr[K_RADJ] = pair;
   {  // tune on work fields and the accumulator (no trace read, image untouched)
     born::RadjStep t{};
-    t.s1 = ctx->d_w[3]; t.s0 = ctx->d_w[2]; t.r1 = ctx->d_w[1]; t.r0 = ctx->d_w[0];
+    t.pair = pair;
+    t.s1 = ctx->d_w[pair ? 2 : 3]; t.s0 = ctx->d_w[pair ? 0 : 2];
+    t.r1 = ctx->d_w[1]; t.r0 = ctx->d_w[0];
     t.vel1 = ctx->d_vel1; t.vel2 = ctx->d_vel2; t.img = ctx->d_acc;
     t.s_prop = 1; t.r_prop = 1; t.src = no_points(); t.amp_pre = ctx->d_vel1; t.pre = 0;
     t.rec = recmap(ctx);
-    CHK(autotune(ctx, K_RADJ, [&](const born::Tune &tu) {
+    CHK(autotune(ctx, kind, [&](const born::Tune &tu) {
       return born::launch_radj_step(geo, tu, t, ctx->stream); }));
   }
-  const born::Tune tu = tuning(ctx, K_RADJ);
-  CHK(zero(ctx, ctx->d_w[0], n));
-  CHK(zero(ctx, ctx->d_w[1], n));
+  const born::Tune tu = tuning(ctx, kind);
+  if (pair) {
+    HIPCHK(born::launch_interleave(ctx->d_w[0], p0, nullptr, n, ctx->stream));
+    HIPCHK(born::launch_interleave(ctx->d_w[2], p1, nullptr, n, ctx->stream));
+  } else {
+    CHK(zero(ctx, ctx->d_w[0], n));
+    CHK(zero(ctx, ctx->d_w[1], n));
+  }
   // cpu_prop.cc:71-95 with _dir = -1 and _jt from the last sourceProp
   const float scale = -1 / (float)ctx->jt_state;
   if (nt > 0) CHK(source_amps(ctx, nt, ctx->jts, 1, scale));
-  float *s_old = p0, *s_cur = p1;
+  float *s_old = pair ? ctx->d_w[0] : p0, *s_cur = pair ? ctx->d_w[2] : p1;
   float *r_old = ctx->d_w[0], *r_cur = ctx->d_w[1];
   born::RadjStep a{};
+  a.pair = pair;
   a.vel1 = ctx->d_vel1;
   a.vel2 = ctx->d_vel2;
   a.img = img;
@@ -1762,6 +1801,10 @@ int born_dev_rtm_adjoint(born_ctx *ctx, int nt, float *p0, float *p1, float *img
     HIPCHK(born::launch_radj_step(geo, sweep(tu, it), a, ctx->stream));
     std::swap(s_old, s_cur);
     std::swap(r_old, r_cur);
+  }
+  if (pair) {  // the state of s goes back to the arrays it came from
+    HIPCHK(born::launch_first_of_pairs(p0, ctx->d_w[0], n, ctx->stream));
+    HIPCHK(born::launch_first_of_pairs(p1, ctx->d_w[2], n, ctx->stream));
   }
   return BORN_OK;
 }
@@ -2241,6 +2284,7 @@ int born_set_autotune(born_ctx *ctx, int on) {
 int born_get_tuning(const born_ctx *ctx, int kernel, int *rows_per_thread,
                     int *waves_per_block, int *zchunk, float *ms) {
   if (!ctx || kernel < 0 || kernel >= K_NUM) return BORN_ERR_ARG;
+  kernel = tuned_slot(ctx, kernel);
   const born::Tune t = tuning(ctx, kernel);
   if (rows_per_thread)
     *rows_per_thread = is_pair(kernel) ? born::kPairShapes[t.shape].ry : born::kShapes[t.shape].ry;
@@ -2262,7 +2306,7 @@ int born_get_tile(const born_ctx *ctx, int kernel, int *tile_x, int *tile_y,
     if (lookahead) *lookahead = 1;
     return BORN_OK;
   }
-  const born::TileShape &ts = born::kShapes[tuning(ctx, kernel).shape];
+  const born::TileShape &ts = born::kShapes[tuning(ctx, tuned_slot(ctx, kernel)).shape];
   if (tile_x) *tile_x = ts.lx * ts.vx;
   if (tile_y) *tile_y = ts.ry * (born::kTX * ts.wy / ts.lx);
   if (cells_per_lane) *cells_per_lane = ts.vx;
@@ -2290,8 +2334,11 @@ int born_set_tuning(born_ctx *ctx, int kernel, int rows_per_thread, int waves_pe
     const born::TileShape &ts = born::kShapes[sh];
     if (ts.ry == rows_per_thread && ts.wy == waves_per_block && ts.vx == cells_per_lane &&
         ts.la == lookahead) {
-      ctx->tune[kernel] = {sh, zchunk};
-      ctx->tune_ms[kernel] = 0.f;  // fixed: the autotuner leaves it
+      for (int k : {kernel, sr_kind(kernel)})
+        if (k >= 0) {
+          ctx->tune[k] = {sh, zchunk};
+          ctx->tune_ms[k] = 0.f;  // fixed: the autotuner leaves it
+        }
       return BORN_OK;
     }
   }
@@ -2327,6 +2374,8 @@ struct born_batch {
   int max_nzi = 1;  // most interior planes of a shot
   std::vector<long long> src0;  // source samples of shot s in d_src ([npts][ntb])
   int npts_total = 0;
+  // four levels, one allocation (d_f[0]); a level of s and r together takes
+  // d_f[0] and d_f[1], or d_f[2] and d_f[3]
   float *d_f[4] = {nullptr, nullptr, nullptr, nullptr};
   float *d_vel = nullptr, *d_model = nullptr, *d_sponge = nullptr, *d_src = nullptr;
   float *d_amp = nullptr;
@@ -2395,7 +2444,7 @@ int batch_step_buffers(born_batch *b, int nt, int rwin) {
 void batch_free(born_batch *b) {
   born_ctx *ctx = b->ctx;
   batch_drop_graph(b);
-  for (int i = 0; i < 4; i++) (void)dev_alloc(ctx, &b->d_f[i], 0);
+  (void)dev_alloc(ctx, &b->d_f[0], 0);
   (void)dev_alloc(ctx, &b->d_vel, 0);
   (void)dev_alloc(ctx, &b->d_model, 0);
   (void)dev_alloc(ctx, &b->d_sponge, 0);
@@ -2424,6 +2473,16 @@ int upload(born_ctx *ctx, T **dst, const std::vector<T> &v) {
   CHK(dev_alloc(ctx, dst, std::max<size_t>(v.size(), 1)));
   if (!v.empty())
     HIPCHK(hipMemcpy(*dst, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+  return BORN_OK;
+}
+
+// the four level buffers, `floats` each at least
+int batch_fields(born_batch *b, size_t floats) {
+  const size_t cap = whole_lines(floats);
+  b->f_cap = 0;
+  CHK(dev_alloc(b->ctx, &b->d_f[0], 4 * cap));
+  for (int i = 1; i < 4; i++) b->d_f[i] = b->d_f[0] + i * cap;
+  b->f_cap = cap;
   return BORN_OK;
 }
 
@@ -2525,8 +2584,7 @@ int batch_build(born_batch *b, int nshots, const born_shot *shots) {
   b->npts_total = (int)(pts.size() / 4);
   CHK(set_device(ctx));
   HIPCHK(hipStreamSynchronize(ctx->stream));
-  for (int i = 0; i < 4; i++) CHK(dev_alloc(ctx, &b->d_f[i], (size_t)cells));
-  b->f_cap = (size_t)cells;
+  CHK(batch_fields(b, (size_t)cells));
   CHK(dev_alloc(ctx, &b->d_vel, (size_t)cells));
   CHK(dev_alloc(ctx, &b->d_model, (size_t)cells));
   for (int s = 0; s < nshots; s++) {
@@ -2578,10 +2636,8 @@ born::BatchFwdStep batch_step(born_batch *b, int it, int jt, int scatter, int st
   born::BatchFwdStep st{};
   born::FwdStep &a = st.a;
   const bool odd = it % 2;
-  a.s1 = b->d_f[odd ? 0 : 1];
-  a.s0 = b->d_f[odd ? 1 : 0];
-  a.r1 = b->d_f[odd ? 2 : 3];
-  a.r0 = b->d_f[odd ? 3 : 2];
+  a.s1 = b->d_f[odd ? 0 : 2];  // s and r together
+  a.s0 = b->d_f[odd ? 2 : 0];
   a.vel = b->d_vel;
   a.model = b->d_model;
   a.src = {b->d_pts, 0};
@@ -2664,9 +2720,7 @@ int born_batch_forward(born_batch *b, int jt, int nt, int scatter) {
   const size_t fneed = split ? ((size_t)b->cells * 3 + 1) / 2 : (size_t)b->cells;
   if (b->f_cap < fneed) {
     batch_drop_graph(b);  // it holds the old buffers
-    b->f_cap = 0;
-    for (int i = 0; i < 4; i++) CHK(dev_alloc(ctx, &b->d_f[i], fneed));
-    b->f_cap = fneed;
+    CHK(batch_fields(b, fneed));
   }
   const born::Taps taps = taps_of(b->coeffs);
   const int rwin = rec_window(nt, b->rec_total);

@@ -637,6 +637,28 @@ __device__ __forceinline__ void ld_vec2(const float2 *p, uint32_t po, uint32_t o
   }
 }
 
+template <int VX>
+__device__ __forceinline__ void ld_pair(const float2 *p, uint32_t po, uint32_t o,
+                                        const float (&)[2], float (&v)[2][VX], uint32_t = 0) {
+  ld_vec2<VX>(p, po, o, v[0], v[1]);
+}
+template <int VX, bool NT = true>
+__device__ __forceinline__ void st_pair(float2 *p, uint32_t po, uint32_t o, const float (&a)[VX],
+                                        const float (&b)[VX], const float (&)[2], uint32_t = 0) {
+  const char *q = adv(p, (uint64_t)po * 8u);
+#pragma unroll
+  for (int h = 0; h < (VX + 1) / 2; h++) {
+    constexpr int N = VX == 1 ? 2 : 4;
+    uint32_t u[N];
+#pragma unroll
+    for (int i = 0; i < N / 2; i++) {
+      u[2 * i] = __float_as_uint(a[2 * h + i]);
+      u[2 * i + 1] = __float_as_uint(b[2 * h + i]);
+    }
+    st_words<NT>(q + 16 * h, o * 8u, u);
+  }
+}
+
 template <int VX, bool NT = true>
 __device__ __forceinline__ void st_vec(float *p, uint32_t po, uint32_t o, const float (&v)[VX],
                                        float, uint32_t = 0) {

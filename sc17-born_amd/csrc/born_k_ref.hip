@@ -1,4 +1,5 @@
-// Launchers of the reference-mode loops: sourceProp and rtmAdjoint steps.
+// Launchers of the reference-mode loops: sourceProp and rtmAdjoint steps (the
+// latter with s and r together: born_k_radj2.hip).
 #include "born_ops.h"
 
 namespace born {
@@ -11,15 +12,12 @@ hipError_t launch_src_step(const Geometry &geo, const Tune &tu, const SrcStep &a
   return launch(geo, tu, op, st);
 }
 
+BORN_RADJ_STEP(extern template, true);
+BORN_RADJ_STEP(template, false);
+
 hipError_t launch_radj_step(const Geometry &geo, const Tune &tu, const RadjStep &a,
                             hipStream_t st) {
-  RadjOp op{};
-  op.s1 = a.s1; op.r1 = a.r1; op.s0 = a.s0; op.r0 = a.r0;
-  op.vel1 = a.vel1; op.vel2 = a.vel2; op.img = a.img;
-  op.s_prop = a.s_prop; op.r_prop = a.r_prop;
-  op.pts = to_points(a.src); op.amp_pre = a.amp_pre; op.pre = a.pre;
-  op.rm = a.rec; op.gin = a.gin; op.nx = geo.nx; op.ny = geo.ny;
-  return launch(geo, tu, op, st);
+  return a.pair ? radj_step<true>(geo, tu, a, st) : radj_step<false>(geo, tu, a, st);
 }
 
 }  // namespace born

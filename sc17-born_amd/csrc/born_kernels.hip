@@ -184,6 +184,8 @@ const TileShape kShapes[kNumShapes] = {
 #define BORN_ALL_TYPES(M, ...) M(__VA_ARGS__, float); M(__VA_ARGS__, __half); M(__VA_ARGS__, Split)
 BORN_ALL_TYPES(BORN_FWD_STEP, extern template, 0);
 BORN_ALL_TYPES(BORN_FWD_STEP, extern template, 1);
+BORN_FWD_STEP_SR(extern template, 0);
+BORN_FWD_STEP_SR(extern template, 1);
 BORN_ALL_TYPES(BORN_SREC_STEP, extern template, 0);
 BORN_ALL_TYPES(BORN_SREC_STEP, extern template, 1);
 BORN_ALL_TYPES(BORN_LAM_STEP, extern template);
@@ -204,9 +206,13 @@ static hipError_t by_storage(int on, F f) {
 
 hipError_t launch_fwd_step(const Geometry &geo, const Tune &tu, const FwdStep &a,
                            hipStream_t st) {
+  if (a.h.on == 0 && a.pair)
+    return a.scatter == 0 ? fwd_step<0, float, true>(geo, tu, a, st)
+                          : fwd_step<1, float, true>(geo, tu, a, st);
   return by_storage(a.h.on, [&](auto t) {
     using T = decltype(t);
-    return a.scatter == 0 ? fwd_step<0, T>(geo, tu, a, st) : fwd_step<1, T>(geo, tu, a, st);
+    return a.scatter == 0 ? fwd_step<0, T, kNarrow<T>>(geo, tu, a, st)
+                          : fwd_step<1, T, kNarrow<T>>(geo, tu, a, st);
   });
 }
 
@@ -247,11 +253,26 @@ hipError_t launch_batch_lam_step(const Taps &taps, const Tune &tu, const BatchLa
                     [&](auto t) { return batch_lam_step<decltype(t)>(taps, tu, b, st); });
 }
 
-// dst[2i] = a[i], dst[2i+1] = b[i]
+// dst[2i] = a[i], dst[2i+1] = b[i] (b null: 0)
 __global__ void interleave_kernel(float2 *dst, const float *a, const float *b, long long n) {
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x)
-    dst[i] = make_float2(a[i], b[i]);
+    dst[i] = make_float2(a[i], b ? b[i] : 0.f);
+}
+
+// dst[i] = src[2i]
+__global__ void first_of_pairs_kernel(float *dst, const float2 *src, long long n) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (long long)gridDim.x * blockDim.x)
+    dst[i] = src[i].x;
+}
+
+hipError_t launch_first_of_pairs(float *dst, const float *src, long long n, hipStream_t st) {
+  if (n <= 0) return hipSuccess;
+  const long long nb = std::min((n + 255) / 256, 65536ll);
+  hipLaunchKernelGGL(first_of_pairs_kernel, dim3((unsigned)nb), dim3(256), 0, st, dst,
+                     (const float2 *)src, n);
+  return hipGetLastError();
 }
 
 hipError_t launch_interleave(float *dst, const float *a, const float *b, long long n,

@@ -62,6 +62,9 @@ struct FwdStep {
   float *rv;  // [nrec] new r at the receiver cells, by first receiver (null: not wanted)
   int scatter;
   Half h;
+  // FP32 levels: s and r together per cell, s1 and s0 hold both (2n floats);
+  // narrow levels always are
+  int pair;
   float *rg;  // FP16 ring block: s ring at 0, r ring at 8, max |model| at 16
   float *hscale;
 };
@@ -115,6 +118,7 @@ struct RadjStep {
   float *s0, *r0;
   const float *vel1, *vel2;
   float *img;
+  int pair;  // s and r together per cell: s1 and s0 hold both (2n floats)
   int s_prop, r_prop;
   SrcPts src;
   const float *amp_pre;
@@ -245,9 +249,11 @@ hipError_t launch_rec_accum(const RecWindow &w, float *tr, const float *rv, hipS
 hipError_t launch_rec_inject(const RecWindow &w, const float *tr, float *gin, bool sum,
                              float scale, hipStream_t st);
 hipError_t launch_fill(float *p, long long n, float v, hipStream_t st);
-// dst (2n floats) = a and b interleaved cell by cell
+// dst (2n floats) = a and b (null: zeros) interleaved cell by cell
 hipError_t launch_interleave(float *dst, const float *a, const float *b, long long n,
                              hipStream_t st);
+// dst = the first field of src (2n floats)
+hipError_t launch_first_of_pairs(float *dst, const float *src, long long n, hipStream_t st);
 hipError_t launch_src_amp(float *amp, int nsteps, int npts, const float *src, int ntsrc,
                           const float *tab, int nsinc, int jt, int ntab, int t_off,
                           float scale, hipStream_t st, int stride = -1);

@@ -54,9 +54,11 @@ constexpr bool kSplit = std::is_same<T, Split>::value;
 // together, the steps run in pairs, the streams take the FP16 cache hints
 template <class T>
 constexpr bool kNarrow = !std::is_same<T, float>::value;
-// two fields stored together: FP16 as __half2, 24-bit as SplitPair
+// two fields stored together: FP32 as float2, FP16 as __half2, 24-bit as
+// SplitPair
 template <class T>
-using PairOf = typename std::conditional<kSplit<T>, SplitPair, __half2>::type;
+using PairOf = typename std::conditional<
+    kNarrow<T>, typename std::conditional<kSplit<T>, SplitPair, __half2>::type, float2>::type;
 
 struct Blk1 {  // one stored field
   PtsBlk pb;
@@ -83,13 +85,20 @@ __device__ __forceinline__ float amp_sum(const Points &pts, const float *amp) {
 // 304^3 175.1 -> 172.6 (207.6 -> 194.1).  The stores keep it in FP32: 304^3
 // 172.4 with, 177.9 without.  FP16 without any: 160^3 38.1 -> 36.1, 224^3 72.8
 // -> 66.9, 304^3 127.9 -> 128.9.
-template <int SCATTER, class T, bool NT = true>
+//
+// PAIR: s and r together per cell.  Half as many streams, twice as long: rows
+// of a level are seldom whole cache lines, and each tile's row ends in two
+// partial ones per stream.  FP32, us per step apart -> together: 160^3 25.2 ->
+// 22.9, 224^3 61.5 -> 51.8, 304^3 173.7 -> 162.9, 203^3 54.6 -> 52.8, 64^3 7.8 ->
+// 7.7; 16 shots of 114-144 x 114-152 x 112 222 -> 188.  FP32 levels stay apart
+// where a kept history or a checkpoint holds the s levels by themselves.
+template <int SCATTER, class T, bool NT = true, bool PAIR = kNarrow<T>>
 struct FwdOp {
   static constexpr bool H = kScaled<T>;
   static constexpr int NF = 2, NPRE = 4, NOUT = 3, NMAX = H ? 2 : 0, REC = 1;
-  // FP16 and 24-bit levels hold s and r together per cell (sr1: level k,
-  // sr0: level k-1, srn: level k+1, the same buffer as sr0 in place)
-  static constexpr bool PAIRED = kNarrow<T>;
+  // s and r together per cell: sr1 level k, sr0 level k-1, srn level k+1, the
+  // same buffer as sr0 in place
+  static constexpr bool PAIRED = PAIR;
   static constexpr bool Q2 = kNarrow<T>;  // steps in pairs (march_tile)
   static constexpr bool DAMP = true;
   const T *__restrict__ s1;
@@ -277,9 +286,13 @@ struct SrcOp {
 };
 
 // ------------------------------------------------------ reference adjoint
+// PAIR: s and r together per cell in s1 and s0, as in the forward (FP32, us per
+// step apart -> together: 160^3 27.9 -> 26.8, 224^3 86.5 -> 77.3, 304^3 223.6 ->
+// 210.6, 203^3 59.7 -> 57.5; 64^3 7.0 -> 7.6).
+template <bool PAIR>
 struct RadjOp {
   static constexpr int NF = 2, NPRE = 5, NOUT = 3, NMAX = 0, REC = 2;
-  static constexpr bool PAIRED = false;
+  static constexpr bool PAIRED = PAIR;
   static constexpr bool Q2 = false;
   static constexpr bool DAMP = true;
   const float *__restrict__ s1;
@@ -309,14 +322,22 @@ struct RadjOp {
   __device__ void ldv(uint32_t, int f, uint32_t po, uint32_t o, float (&v)[VX]) const {
     ld_vec<VX>(f == 0 ? s1 : r1, po, o, 1.f, v);
   }
+  template <int VX>
+  __device__ void ldv2(uint32_t, uint32_t po, uint32_t o, float (&v)[2][VX]) const {
+    ld_vec2<VX>((const float2 *)s1, po, o, v[0], v[1]);
+  }
   __device__ SrcPln plane(uint32_t blk, int z) const {
     return {points_on_plane(pts, blk, z), ldc(rm.plane_slot, z)};
   }
   template <int VX>
   __device__ void prefetchv(uint32_t, float (&p)[NPRE][VX], uint32_t po,
                             uint32_t o) const {
-    ld_vec<VX>(s0, po, o, 1.f, p[0]);
-    ld_vec<VX>(r0, po, o, 1.f, p[1]);
+    if constexpr (PAIRED) {
+      ld_vec2<VX>((const float2 *)s0, po, o, p[0], p[1]);
+    } else {
+      ld_vec<VX>(s0, po, o, 1.f, p[0]);
+      ld_vec<VX>(r0, po, o, 1.f, p[1]);
+    }
     ld_vec<VX>(vel1, po, o, 1.f, p[2]);
     ld_vec<VX>(vel2, po, o, 1.f, p[3]);
     ld_vec<VX>(img, po, o, 1.f, p[4]);
@@ -326,8 +347,13 @@ struct RadjOp {
                          const float (&out)[NOUT][VX]) const {
     // no hint: every array here is read again by the next step (304^3 227.9 ->
     // 223.4 us, 160^3 29.4 -> 27.9; with the hint on the loads too, 160^3 35)
-    if (s_prop) st_vec<VX, false>(s0, po, o, out[0], 1.f);
-    st_vec<VX, false>(r0, po, o, out[1], 1.f);
+    if constexpr (PAIRED) {  // out[0] is the old s when s stands still
+      const float one[2] = {1.f, 1.f};
+      st_pair<VX, false>((float2 *)s0, po, o, out[0], out[1], one);
+    } else {
+      if (s_prop) st_vec<VX, false>(s0, po, o, out[0], 1.f);
+      st_vec<VX, false>(r0, po, o, out[1], 1.f);
+    }
     st_vec<VX, false>(img, po, o, out[2], 1.f);
   }
   __device__ void cell(uint32_t, const SrcPln &pl, const CellArgs &c, const float *lap,
@@ -526,7 +552,7 @@ template <int SCATTER, class T>
 struct BatchFwd {
   // without the non-temporal hint: it slowed the batch (32 windowed shots)
   // by about 5 % where it sped up single shots
-  using Op = FwdOp<SCATTER, T, false>;
+  using Op = FwdOp<SCATTER, T, false, true>;
   Op base;
   const float *sponge;
   float *rings;
@@ -768,9 +794,9 @@ hipError_t launch_batch(const Taps &taps, const Tune &tu, const BatchCommon &b,
 // instantiated explicitly, each in one translation unit (born_k_*.hip, built
 // in parallel); born_kernels.hip declares them extern and dispatches.
 
-template <int SCATTER, class T>
+template <int SCATTER, class T, bool PAIR>
 hipError_t fwd_step(const Geometry &geo, const Tune &tu, const FwdStep &a, hipStream_t st) {
-  FwdOp<SCATTER, T> op{};
+  FwdOp<SCATTER, T, true, PAIR> op{};
   op.s1 = as<T>(a.s1); op.r1 = as<T>(a.r1); op.s0 = as<T>(a.s0); op.r0 = as<T>(a.r0);
   op.s_new = as<T>(a.s_new ? a.s_new : a.s0);
   op.sr1 = (const PairOf<T> *)a.s1; op.sr0 = (const PairOf<T> *)a.s0;
@@ -782,6 +808,17 @@ hipError_t fwd_step(const Geometry &geo, const Tune &tu, const FwdStep &a, hipSt
   op.rg = a.rg; op.slots = pack_slots(a.h.sl);
   op.gain = a.h.gain; op.tapsum = a.h.tapsum; op.hscale = a.hscale;
   op.nlev = (uint32_t)geo.nx * geo.ny * geo.nz;
+  return launch(geo, tu, op, st);
+}
+
+template <bool PAIR>
+hipError_t radj_step(const Geometry &geo, const Tune &tu, const RadjStep &a, hipStream_t st) {
+  RadjOp<PAIR> op{};
+  op.s1 = a.s1; op.r1 = a.r1; op.s0 = a.s0; op.r0 = a.r0;
+  op.vel1 = a.vel1; op.vel2 = a.vel2; op.img = a.img;
+  op.s_prop = a.s_prop; op.r_prop = a.r_prop;
+  op.pts = to_points(a.src); op.amp_pre = a.amp_pre; op.pre = a.pre;
+  op.rm = a.rec; op.gin = a.gin; op.nx = geo.nx; op.ny = geo.ny;
   return launch(geo, tu, op, st);
 }
 
@@ -856,8 +893,14 @@ hipError_t batch_lam_step(const Taps &taps, const Tune &tu, const BatchLamStep &
 }
 
 // the instantiations, one translation unit each (F: template or extern template)
-#define BORN_FWD_STEP(F, S, T) \
-  F hipError_t fwd_step<S, T>(const Geometry &, const Tune &, const FwdStep &, hipStream_t)
+#define BORN_FWD_STEP(F, S, T)                                                          \
+  F hipError_t fwd_step<S, T, kNarrow<T>>(const Geometry &, const Tune &, const FwdStep &, \
+                                          hipStream_t)
+// FP32 levels of s and r together
+#define BORN_FWD_STEP_SR(F, S) \
+  F hipError_t fwd_step<S, float, true>(const Geometry &, const Tune &, const FwdStep &, hipStream_t)
+#define BORN_RADJ_STEP(F, PAIR) \
+  F hipError_t radj_step<PAIR>(const Geometry &, const Tune &, const RadjStep &, hipStream_t)
 #define BORN_SREC_STEP(F, S, T) \
   F hipError_t srec_step<S, T>(const Geometry &, const Tune &, const SrecStep &, hipStream_t)
 #define BORN_LAM_STEP(F, T) \
