@@ -27,6 +27,7 @@
 
 #include "born_hip.h"
 #include "born_launch.h"
+#include "host_copy.h"
 #include "host_par.h"
 
 using born::Geometry;
@@ -35,6 +36,7 @@ struct born_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   std::string err;
+  born::HostCopy copy;  // large results to the caller's arrays
 
   bool have_space = false;
   int nx = 0, ny = 0, nz = 0;
@@ -814,8 +816,7 @@ int traces_out(born_ctx *ctx, float *h) {
   const size_t bytes = (size_t)ctx->nrec * ctx->nt_rec * sizeof(float);
   HIPCHK(born::launch_transpose(ctx->d_tr2, ctx->d_tr, ctx->nt_rec, ctx->nrec,
                                 ctx->stream));
-  HIPCHK(hipMemcpyAsync(h, ctx->d_tr2, bytes, hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
+  HIPCHK(ctx->copy.out(h, ctx->d_tr2, bytes, ctx->stream));
   return BORN_OK;
 }
 
@@ -1148,6 +1149,7 @@ int born_destroy(born_ctx *ctx) {
                   ctx->d_ring,  ctx->d_hscale, ctx->d_ckring, ctx->d_vm};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
+  ctx->copy.release();
   (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return BORN_OK;
@@ -2164,9 +2166,8 @@ int born_source_prop(born_ctx *ctx, int nx, int ny, int nz, int damp, int get_la
   HIPCHK(hipMemcpyAsync(ctx->d_p0, p0, B, hipMemcpyHostToDevice, ctx->stream));
   HIPCHK(hipMemcpyAsync(ctx->d_p1, p1, B, hipMemcpyHostToDevice, ctx->stream));
   CHK(born_dev_source_prop(ctx, jts, nt, ctx->d_p0, ctx->d_p1));
-  HIPCHK(hipMemcpyAsync(p0, ctx->d_p0, B, hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipMemcpyAsync(p1, ctx->d_p1, B, hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
+  HIPCHK(ctx->copy.out(p0, ctx->d_p0, B, ctx->stream));
+  HIPCHK(ctx->copy.out(p1, ctx->d_p1, B, ctx->stream));
   return BORN_OK;
 }
 
@@ -2189,10 +2190,9 @@ int born_rtm_adjoint(born_ctx *ctx, int n1, int n2, int n3, int jtd, float *p0,
   HIPCHK(hipMemcpyAsync(ctx->d_img, img, B, hipMemcpyHostToDevice, ctx->stream));
   CHK(traces_in(ctx, ctx->h_rec));
   CHK(born_dev_rtm_adjoint(ctx, nt, ctx->d_p0, ctx->d_p1, ctx->d_img, ctx->d_tr));
-  HIPCHK(hipMemcpyAsync(img, ctx->d_img, B, hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipMemcpyAsync(p0, ctx->d_p0, B, hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipMemcpyAsync(p1, ctx->d_p1, B, hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
+  HIPCHK(ctx->copy.out(img, ctx->d_img, B, ctx->stream));
+  HIPCHK(ctx->copy.out(p0, ctx->d_p0, B, ctx->stream));
+  HIPCHK(ctx->copy.out(p1, ctx->d_p1, B, ctx->stream));
   return BORN_OK;
 }
 
@@ -2208,8 +2208,7 @@ int born_adjoint_exact(born_ctx *ctx, int n1, int n2, int n3, int jt, const floa
   HIPCHK(hipMemcpyAsync(ctx->d_img, img, B, hipMemcpyHostToDevice, ctx->stream));
   CHK(traces_in(ctx, rec));
   CHK(born_dev_adjoint_exact(ctx, jt, nt, scatter, ctx->d_tr, ctx->d_img));
-  HIPCHK(hipMemcpyAsync(img, ctx->d_img, B, hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
+  HIPCHK(ctx->copy.out(img, ctx->d_img, B, ctx->stream));
   return BORN_OK;
 }
 
@@ -2803,9 +2802,7 @@ int born_batch_traces(born_batch *b, int shot, float *rec) {
   CHK(set_device(ctx));
   const born::ShotDesc &d = b->desc[shot];
   HIPCHK(born::launch_transpose(b->d_tmp, b->d_tr + d.tr0, b->ntb, d.nrec, ctx->stream));
-  HIPCHK(hipMemcpyAsync(rec, b->d_tmp, (size_t)d.nrec * b->ntb * sizeof(float),
-                        hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
+  HIPCHK(ctx->copy.out(rec, b->d_tmp, (size_t)d.nrec * b->ntb * sizeof(float), ctx->stream));
   return BORN_OK;
 }
 
@@ -3116,9 +3113,8 @@ int born_batch_image(born_batch *b, int shot, float *img) {
   if (!b->d_img) return fail(ctx, BORN_ERR_STATE, "no batch adjoint has run");
   CHK(set_device(ctx));
   const born::ShotDesc &d = b->desc[shot];
-  HIPCHK(hipMemcpyAsync(img, b->d_img + d.cell0, (size_t)d.nx * d.ny * d.nz * sizeof(float),
-                        hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
+  HIPCHK(ctx->copy.out(img, b->d_img + d.cell0, (size_t)d.nx * d.ny * d.nz * sizeof(float),
+                       ctx->stream));
   return BORN_OK;
 }
 
