@@ -1404,9 +1404,17 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
   ctx->jt_state = jt;
   const Geometry geo = geometry(ctx);
   // FP32 levels of s and r together (see FwdOp), unless s levels are wanted by
-  // themselves: in the history (scatter 0), in checkpoints, in a two-step
-  // launch; a segment history's gaps hold r alone, too
-  const bool pair = !half && !try_pairs && ckS == 0 && (!hist || (scatter == 1 && !ctx->seg_gap));
+  // themselves: in checkpoints, in a two-step launch, in a history with gaps
+  // (which hold r alone).  With scatter 0 the levels of s can be those of the
+  // history, which saves writing s twice, or stay with r: faster while the
+  // levels, velocity and model (24 bytes per cell) about fit the 256 MB
+  // memory-side cache, from which the history then takes nothing.  us per step
+  // in the history -> with r: 64^3 8.3 -> 8.3, 128^3 20.1 -> 17.2, 160^3 27.4 ->
+  // 24.1, 203^3 66.2 -> 58.3, 224^3 65.6 -> 56.0, 240^3 110.5 -> 104.0; 256^3
+  // 96.8 -> 106.7, 304^3 172.6 -> 185.8
+  const bool pair = !half && !try_pairs && ckS == 0 &&
+                    (!hist || (!ctx->seg_gap &&
+                               (scatter == 1 || (n >= 1 << 19 && n <= 14000000))));
   const int fkind = fwd_kind(ctx->storage, scatter);
   const int kind = pair ? sr_kind(fkind) : fkind;
   if (!half) ctx->tuned_sr[fkind] = pair;
@@ -1430,7 +1438,7 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
     // launch after launch time up to 20 % faster than the steps run, and
     // pick another tile.  Else the history level written beside the
     // in-place s.
-    const bool rotate = hist && scatter == 0 && !half && nt >= 3;
+    const bool rotate = hist && scatter == 0 && !half && !pair && nt >= 3;
     if (!rotate) t.hist = hist;
     int lev = 0;
     CHK(autotune(ctx, kind, [&](const born::Tune &tu) {
@@ -1439,6 +1447,9 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
         t.s1 = seg_level(ctx, lev + 1);
         t.s_new = seg_level(ctx, lev + 2);
         lev = (lev + 1) % (nt - 2);
+      } else if (hist && pair) {  // likewise the next level each launch
+        t.hist = seg_level(ctx, lev);
+        lev = (lev + 1) % nt;
       }
       return born::launch_fwd_step(geo, tu, t, ctx->stream); }));
   }
@@ -1578,7 +1589,7 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
   // write per cell less than a separate s buffer and history.  (FP16 levels
   // keep s and r together as one __half2 per cell in sb[], and the history
   // is written apart.)
-  const bool s_in_hist = hist && scatter == 0 && !half;
+  const bool s_in_hist = hist && scatter == 0 && !half && !pair;
   // checkpoint plan: levels it and it-1 saved before step it at segment
   // starts it = c L (c = 1..S-1); from klast on the scatter operands go to
   // the segment history (scatter 0: the s levels themselves, level j > klast

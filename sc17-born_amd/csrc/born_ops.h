@@ -91,7 +91,7 @@ __device__ __forceinline__ float amp_sum(const Points &pts, const float *amp) {
 // partial ones per stream.  FP32, us per step apart -> together: 160^3 25.2 ->
 // 22.9, 224^3 61.5 -> 51.8, 304^3 173.7 -> 162.9, 203^3 54.6 -> 52.8, 64^3 7.8 ->
 // 7.7; 16 shots of 114-144 x 114-152 x 112 222 -> 188.  FP32 levels stay apart
-// where a kept history or a checkpoint holds the s levels by themselves.
+// where s levels are wanted by themselves (born_dev_forward).
 template <int SCATTER, class T, bool NT = true, bool PAIR = kNarrow<T>>
 struct FwdOp {
   static constexpr bool H = kScaled<T>;
