@@ -78,7 +78,7 @@ __device__ __forceinline__ float amp_sum(const Points &pts, const float *amp) {
 // ---------------------------------------------------------------- forward
 // NT: the single-shot forward: non-temporal hint on the FP32 and 24-bit
 // stores, velocity and model as one stream (the shot batch: see BatchFwd).
-// The loads take no hint: what a step reads the next one reads or overwrites,
+// The loads take no hint (but see s0): what a step reads the next one reads or overwrites,
 // and a load with the hint leaves nothing in the 256 MB memory-side cache.
 // FP32, us per step with the hint on the pointwise loads -> without: 160^3
 // 31.6 -> 26.4 (dV scatter 35.5 -> 26.1), 224^3 73.7 -> 63.9 (83.7 -> 61.7),
@@ -195,7 +195,10 @@ struct FwdOp {
         p[1][v] = sr[1][v];
       }
     } else {
-      ld_vec<VX>(s0, po, o, b.io[0], p[0], nlev);
+      // s0 alone takes the hint: levels apart are those of a kept history, whose
+      // oldest one no step reads again (304^3 169.9 -> 167.7 us, 352^3 266.1 ->
+      // 260.9)
+      ld_vec<VX, true>(s0, po, o, b.io[0], p[0], nlev);
       ld_vec<VX>(r0, po, o, b.io[1], p[1], nlev);
     }
     if constexpr (NT) {
