@@ -1404,17 +1404,18 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
   ctx->jt_state = jt;
   const Geometry geo = geometry(ctx);
   // FP32 levels of s and r together (see FwdOp), unless s levels are wanted by
-  // themselves: in checkpoints, in a two-step launch, in a history with gaps
-  // (which hold r alone).  With scatter 0 the levels of s can be those of the
+  // themselves: in checkpoints, in a two-step launch.  With scatter 0 the levels of s can be those of the
   // history, which saves writing s twice, or stay with r: faster while the
   // levels, velocity and model (24 bytes per cell) about fit the 256 MB
   // memory-side cache, from which the history then takes nothing.  us per step
   // in the history -> with r: 64^3 8.3 -> 8.3, 128^3 20.1 -> 17.2, 160^3 27.4 ->
   // 24.1, 203^3 66.2 -> 58.3, 224^3 65.6 -> 56.0, 240^3 110.5 -> 104.0; 256^3
-  // 96.8 -> 106.7, 304^3 172.6 -> 185.8
+  // 96.8 -> 106.7, 304^3 172.6 -> 185.8.  A history with gaps (of more than 32
+  // GiB) places levels of r alone, which is worth 2 % at 224^3 in turn: 160^3
+  // 27.2 -> 25.1, 203x187x221 65.8 -> 56.7, 224^3 dV 63.8 -> 65.2
+  const bool mid = n >= 1 << 19 && n <= (ctx->seg_gap ? 10000000 : 14000000);
   const bool pair = !half && !try_pairs && ckS == 0 &&
-                    (!hist || (!ctx->seg_gap &&
-                               (scatter == 1 || (n >= 1 << 19 && n <= 14000000))));
+                    (!hist || mid || (scatter == 1 && !ctx->seg_gap));
   const int fkind = fwd_kind(ctx->storage, scatter);
   const int kind = pair ? sr_kind(fkind) : fkind;
   if (!half) ctx->tuned_sr[fkind] = pair;
@@ -1475,7 +1476,8 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
   // history, level it - klast in the last segment of a checkpoint plan;
   // before klast (s in the work buffers) a window of its own, index ngaps.
   const int klast = ckS > 1 ? (ckS - 1) * ckL : nt;
-  const bool place = ctx->place_mode && ctx->seg_gap && !use_pairs && (hist || ckS > 1);
+  const bool place =
+      ctx->place_mode && ctx->seg_gap && !use_pairs && !pair && (hist || ckS > 1);
   const int wwork = hist ? 0 : 1;  // the window of steps that write no history level
   auto window_of = [&](int it) {
     const long long lv = hist ? it : it >= klast ? it - klast : -1;
