@@ -72,16 +72,22 @@ def test_shapes_give_the_same_bits(pyborn, shape, storage):
 @pytest.mark.parametrize("scatter", [0, 1])
 @pytest.mark.parametrize("n", [(64, 64, 127), (64, 64, 128), (97, 75, 74)])
 def test_levels_together_and_apart(pyborn, n, scatter):
-    # 2^19 cells are the least of a kept history whose s levels stay with r;
-    # one with gaps (short windows) has s and r apart, no history together
+    # 2^19 cells are the least of a kept history whose s levels stay with r.
+    # Without a history s and r are together, with a checkpoint plan apart;
+    # with gaps in the history (short windows) the size decides
     c = make_case(*n, nt=24, nbound=8, src_z=9, rec_z=7, seed=5)
     w = np.random.default_rng(3).standard_normal((c.nrec, c.ntb)).astype(np.float32)
     out = []
-    for keep, gaps in ((False, False), (True, False), (True, True)):
+    F = 4 * c.nx * c.ny * c.nz
+    for form in ("no history", "history", "gaps", "checkpoints"):
         H = _prop(pyborn, c)
-        if gaps:
-            H.set_placement("timed", 10 * 4 * c.nx * c.ny * c.nz)
-        out.append(_pair(H, c, w, scatter, keep))
+        if form == "gaps":
+            H.set_placement("timed", 10 * F)
+        if form == "checkpoints":
+            H.set_checkpoint_budget(16 * F)
+        out.append(_pair(H, c, w, scatter, form != "no history"))
+        if form == "checkpoints":
+            assert H.last_checkpoint_plan()[0] >= 2
         H.close()
     for got in out[1:]:
         assert np.array_equal(got[0], out[0][0]) and np.array_equal(got[1], out[0][1])
