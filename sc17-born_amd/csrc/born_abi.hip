@@ -1404,8 +1404,9 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
   ctx->jt_state = jt;
   const Geometry geo = geometry(ctx);
   // FP32 levels of s and r together (see FwdOp), unless s levels are wanted by
-  // themselves: in checkpoints, in a two-step launch.  With scatter 0 the levels of s can be those of the
-  // history, which saves writing s twice, or stay with r: faster while the
+  // themselves: in checkpoints, in a two-step launch.  With scatter 0 the
+  // levels of s can be those of the history, which saves writing s twice, or
+  // stay with r: faster while the
   // levels, velocity and model (24 bytes per cell) about fit the 256 MB
   // memory-side cache, from which the history then takes nothing.  us per step
   // in the history -> with r: 64^3 8.3 -> 8.3, 128^3 20.1 -> 17.2, 160^3 27.4 ->
