@@ -686,6 +686,7 @@ __device__ __forceinline__ void st_vec(__half *p, uint32_t po, uint32_t o,
 // plane.  Op supplies (all const):
 //   static constexpr int NF, NPRE, NOUT, NMAX; static constexpr bool DAMP;
 //   static constexpr int REC;                   receivers: 0 none, 1 read, 2 injected
+//   static constexpr bool LEAN;                 Laplacians row by row, field by field
 //   Blk block(x0, x1, y0, y1, z0, z1);          uniform per-block state
 //   void first(const Blk&);                     (NMAX > 0) once per launch
 //   ldv<VX>(const Blk&, int f, uint32_t po, uint32_t o, float (&v)[VX])
@@ -786,7 +787,7 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
   constexpr int NHALO = NYH + NXH;
   constexpr int HPT = (NHALO + NT - 1) / NT;
   uint32_t hoff[HPT];
-  short hr[HPT], hc[HPT], hs[HPT];
+  int ht[HPT];  // the unit's place in an LDS tile
   bool hv[HPT];
 #pragma unroll
   for (int k = 0; k < HPT; k++) {
@@ -803,9 +804,7 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
       lr = kH + hh / (2 * XU);
       lc = c < XU ? VX * c : kH + TW + VX * (c - XU);
     }
-    hr[k] = (short)lr;
-    hs[k] = (short)min(h, NHALO - 1);
-    hc[k] = (short)lc;
+    ht[k] = lr * LW + lc;
     const int gy = min(max(y0 - kH + lr, 0), g.ny - 1);
     const int gx = min(max(x0 - kH + lc, 0), g.nx - VX);
     hoff[k] = (uint32_t)gy * g.nx + gx;
@@ -898,7 +897,7 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
       for (int k = 0; k < HPT; k++)
 #pragma unroll
         for (int f = 0; f < NF; f++)
-          if (hv[k]) st_lds<VX>(stage[p][f][hs[k]], h[p][k][f]);
+          if (hv[k]) st_lds<VX>(stage[p][f][(int)threadIdx.x + k * NT], h[p][k][f]);
   }
 
   // The new values of a step are stored at the start of the next step,
@@ -933,8 +932,10 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
 #pragma unroll
       for (int k = 0; k < HPT; k++) {
         float h[VX];
-        ld_lds<VX>(stage[ss][f][hs[k]], h);
-        if (hv[k]) st_lds<VX>(&tile[sl][f][hr[k]][hc[k]], h);
+        if (hv[k]) {
+          ld_lds<VX>(stage[ss][f][(int)threadIdx.x + k * NT], h);
+          st_lds<VX>(&tile[sl][f][0][0] + ht[k], h);
+        }
       }
 #pragma unroll
       for (int j = 0; j < RY; j++) {
@@ -962,7 +963,7 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
         for (int v = 0; v < VX; v++) q[f][j][v][2 * kH + R] = lead[b][f][j][v];
 #pragma unroll
       for (int k = 0; k < HPT; k++)
-        if (hv[k]) st_lds<VX>(stage[ss][f][hs[k]], hl[b][f][k]);
+        if (hv[k]) st_lds<VX>(stage[ss][f][(int)threadIdx.x + k * NT], hl[b][f][k]);
     }
     flush();
     issue(z + D, bn);
@@ -992,10 +993,19 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
     // thread's RY consecutive rows is read from LDS once per field (kH
     // rows either side; the thread's own rows come from its z queues) and
     // shared by the RY cells.
+    // LEAN ops skip the rows outside the domain and finish a field before the
+    // next: left to itself the compiler issues the LDS reads of every row and
+    // field together and holds them all.  Registers of a lane and wavefronts of
+    // a SIMD, without -> with: FP32 forward with s and r apart, 2 x 4, 152 and 3
+    // -> 113 and 4; FP16 forward, 2 x 8 with two planes of lookahead, 162 and 3
+    // -> 127 and 4; 25 of 50 kernels that spilled no longer do.  us per step:
+    // FP32 forward 304^3, 1000 levels kept, 159 -> 154; FP16 forward 304^3 124
+    // -> 114, 480x448x416 411 -> 380.
     const int lr0 = kH + RY * ty, lc = kH + VX * tx;
     float lap[RY][VX][NF];
 #pragma unroll
     for (int f = 0; f < NF; f++) {
+      if (Op::LEAN && f > 0) __builtin_amdgcn_sched_barrier(0);
       float col[RY + 2 * kH][VX];
 #pragma unroll
       for (int i = 0; i < kH; i++) {
@@ -1008,6 +1018,7 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
         for (int v = 0; v < VX; v++) col[kH + j][v] = q[f][j][v][kH + R];
 #pragma unroll
       for (int j = 0; j < RY; j++) {
+        if (Op::LEAN && !in[j]) continue;
         // the row from lc - 4 to lc + VX + 3
         float xs[2 * kH + VX];
 #pragma unroll
