@@ -611,6 +611,7 @@ int ensure_work(born_ctx *ctx) {
   const size_t need = work_floats(ctx);
   if (ctx->w_cap < need) {
     ctx->w_cap = 0;
+    for (int i = 1; i < 4; i++) ctx->d_w[i] = nullptr;  // parts of d_w[0]
     CHK(dev_alloc(ctx, &ctx->d_w[0], 4 * need));
     for (int i = 1; i < 4; i++) ctx->d_w[i] = ctx->d_w[0] + i * need;
     ctx->w_cap = need;
@@ -1185,8 +1186,9 @@ int born_create_space(born_ctx *ctx, float d1, float d2, float d3, float bc_a,
   if (resized) {
     // every buffer of the old cell count goes, the two-step levels included
     // (ensure_work / ensure_pair_work only allocate a missing buffer)
-    CHK(dev_alloc(ctx, &ctx->d_w[0], 0));
+    for (int i = 1; i < 4; i++) ctx->d_w[i] = nullptr;  // parts of d_w[0]
     ctx->w_cap = 0;
+    CHK(dev_alloc(ctx, &ctx->d_w[0], 0));
     for (int i = 0; i < 4; i++) CHK(dev_alloc(ctx, &ctx->d_w2[i], 0));
     CHK(dev_alloc(ctx, &ctx->d_img, 0));
     CHK(dev_alloc(ctx, &ctx->d_acc, 0));
@@ -2489,10 +2491,14 @@ int upload(born_ctx *ctx, T **dst, const std::vector<T> &v) {
   return BORN_OK;
 }
 
-// the four level buffers, `floats` each at least
+// the four level buffers, `floats` each at least.  A call that wants more of
+// them than there is memory for leaves none, and the next call takes its own.
 int batch_fields(born_batch *b, size_t floats) {
+  if (b->f_cap >= floats) return BORN_OK;
   const size_t cap = whole_lines(floats);
+  batch_drop_graph(b);  // it holds the old buffers
   b->f_cap = 0;
+  for (int i = 1; i < 4; i++) b->d_f[i] = nullptr;  // parts of d_f[0]
   CHK(dev_alloc(b->ctx, &b->d_f[0], 4 * cap));
   for (int i = 1; i < 4; i++) b->d_f[i] = b->d_f[0] + i * cap;
   b->f_cap = cap;
@@ -2731,10 +2737,7 @@ int born_batch_forward(born_batch *b, int jt, int nt, int scatter) {
                 "24-bit storage needs fewer than 715,827,882 cells per shot");
   // 24-bit levels of two fields need 6 bytes per cell
   const size_t fneed = split ? ((size_t)b->cells * 3 + 1) / 2 : (size_t)b->cells;
-  if (b->f_cap < fneed) {
-    batch_drop_graph(b);  // it holds the old buffers
-    CHK(batch_fields(b, fneed));
-  }
+  CHK(batch_fields(b, fneed));
   const born::Taps taps = taps_of(b->coeffs);
   const int rwin = rec_window(nt, b->rec_total);
   CHK(batch_step_buffers(b, nt, rwin));
@@ -2861,6 +2864,7 @@ int born_batch_adjoint_exact(born_batch *b, int jt, int nt, int scatter) {
   CHK(ensure(ctx, &b->d_img, &b->img_cap, (size_t)cells));
   CHK(zero(ctx, b->d_img, cells));
   if (nt == 0) return BORN_OK;
+  CHK(batch_fields(b, (size_t)cells));  // (a forward may have left none)
   const int rwin = rec_window(nt, b->rec_total);
   CHK(batch_step_buffers(b, nt, rwin));
   const born::Taps taps = taps_of(b->coeffs);
