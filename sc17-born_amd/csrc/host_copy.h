@@ -87,8 +87,10 @@ class HostCopy {
   // announces a chunk when its transfer is complete, with the next one under
   // way; the threads take the pieces in order.  No thread waits for a chunk
   // that the calling thread could not reach: a slot is free once pieces of
-  // announced chunks are copied.  An error stops the threads.  *ran: false if
-  // no thread could be started (nothing was written to host).
+  // announced chunks are copied.  The threads are started when the first chunk
+  // has arrived: until then the stream may have a whole shot's steps to run,
+  // and they would poll for it.  An error stops them.  *ran: false if no thread
+  // could be started (nothing was written to host).
   hipError_t staged(char *host, const char *dev, size_t bytes, hipStream_t stream, bool *ran) {
     const long n = (long)((bytes + kSlot - 1) / kSlot);
     const long pieces = (long)((bytes + kPiece - 1) / kPiece);
@@ -116,26 +118,31 @@ class HostCopy {
     };
     std::vector<std::atomic<int>> done;
     std::vector<std::thread> pool;
-    try {
-      done = std::vector<std::atomic<int>>(n);
-      pool.reserve(kThreads);
-      const int want = std::min<int>(kThreads, (int)born_par::threads());
-      while ((int)pool.size() < want) pool.emplace_back(work, done.data());
-    } catch (const std::exception &) {
-      if (pool.empty()) return hipSuccess;
-    }
-    *ran = true;
-    for (long i = 0; i <= n && err == hipSuccess; i++) {
-      if (i < n) {
-        if (i >= kSlots)
-          while (done[i - kSlots].load(std::memory_order_acquire) < kPieces)
-            std::this_thread::yield();
+    auto start = [&]() {
+      try {
+        done = std::vector<std::atomic<int>>(n);
+        pool.reserve(kThreads);
+        const int want = std::min<int>(kThreads, (int)born_par::threads());
+        while ((int)pool.size() < want) pool.emplace_back(work, done.data());
+      } catch (const std::exception &) {
+      }
+      return !pool.empty();
+    };
+    for (long i = 0; i < std::min(n, kSlots) && err == hipSuccess; i++) issue(i);
+    for (long i = 1; i <= n && err == hipSuccess; i++) {
+      if (i >= kSlots && i < n) {
+        while (done[i - kSlots].load(std::memory_order_acquire) < kPieces)
+          std::this_thread::yield();
         issue(i);
+        if (err != hipSuccess) break;
       }
-      if (i > 0 && err == hipSuccess) {
-        err = hipEventSynchronize(ev_[(i - 1) % kSlots]);
-        if (err == hipSuccess) arrived.store(i, std::memory_order_release);
+      err = hipEventSynchronize(ev_[(i - 1) % kSlots]);
+      if (err != hipSuccess) break;
+      if (i == 1) {
+        *ran = start();
+        if (!*ran) return hipSuccess;
       }
+      arrived.store(i, std::memory_order_release);
     }
     if (err != hipSuccess) stop.store(true);
     for (std::thread &t : pool) t.join();
