@@ -11,8 +11,10 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstring>
 #include <exception>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -87,16 +89,22 @@ class HostCopy {
   // announces a chunk when its transfer is complete, with the next one under
   // way; the threads take the pieces in order.  No thread waits for a chunk
   // that the calling thread could not reach: a slot is free once pieces of
-  // announced chunks are copied.  The threads are started when the first chunk
-  // has arrived: until then the stream may have a whole shot's steps to run,
-  // and they would poll for it.  An error stops them.  *ran: false if no thread
-  // could be started (nothing was written to host).
+  // announced chunks are copied.  For the first chunk the threads sleep: the
+  // stream may have a whole shot's steps to run before it.  An error stops the
+  // threads.  *ran: false if none could be started (nothing was written to
+  // host).
   hipError_t staged(char *host, const char *dev, size_t bytes, hipStream_t stream, bool *ran) {
     const long n = (long)((bytes + kSlot - 1) / kSlot);
     const long pieces = (long)((bytes + kPiece - 1) / kPiece);
     std::atomic<long> next{0}, arrived{0};
     std::atomic<bool> stop{false};
+    std::mutex m;
+    std::condition_variable first;  // a chunk has arrived, or stop
     auto work = [&, host](std::atomic<int> *done) {
+      {
+        std::unique_lock<std::mutex> lock(m);
+        first.wait(lock, [&] { return arrived.load() > 0 || stop.load(); });
+      }
       for (long p; (p = next.fetch_add(1)) < pieces;) {
         const long c = p / kPieces;
         while (c >= arrived.load(std::memory_order_acquire)) {
@@ -118,15 +126,22 @@ class HostCopy {
     };
     std::vector<std::atomic<int>> done;
     std::vector<std::thread> pool;
-    auto start = [&]() {
-      try {
-        done = std::vector<std::atomic<int>>(n);
-        pool.reserve(kThreads);
-        const int want = std::min<int>(kThreads, (int)born_par::threads());
-        while ((int)pool.size() < want) pool.emplace_back(work, done.data());
-      } catch (const std::exception &) {
+    try {
+      done = std::vector<std::atomic<int>>(n);
+      pool.reserve(kThreads);
+      const int want = std::min<int>(kThreads, (int)born_par::threads());
+      while ((int)pool.size() < want) pool.emplace_back(work, done.data());
+    } catch (const std::exception &) {
+      if (pool.empty()) return hipSuccess;
+    }
+    *ran = true;
+    // wakes the threads with a change that they wait for
+    auto wake = [&](auto change) {
+      {
+        std::lock_guard<std::mutex> lock(m);
+        change();
       }
-      return !pool.empty();
+      first.notify_all();
     };
     for (long i = 0; i < std::min(n, kSlots) && err == hipSuccess; i++) issue(i);
     for (long i = 1; i <= n && err == hipSuccess; i++) {
@@ -138,13 +153,12 @@ class HostCopy {
       }
       err = hipEventSynchronize(ev_[(i - 1) % kSlots]);
       if (err != hipSuccess) break;
-      if (i == 1) {
-        *ran = start();
-        if (!*ran) return hipSuccess;
-      }
-      arrived.store(i, std::memory_order_release);
+      if (i == 1)
+        wake([&] { arrived.store(1); });
+      else
+        arrived.store(i, std::memory_order_release);
     }
-    if (err != hipSuccess) stop.store(true);
+    if (err != hipSuccess) wake([&] { stop.store(true); });
     for (std::thread &t : pool) t.join();
     return err;
   }
