@@ -29,6 +29,7 @@
 #include "born_launch.h"
 #include "host_copy.h"
 #include "host_par.h"
+#include "tune_search.h"
 
 using born::Geometry;
 
@@ -360,25 +361,11 @@ born::Tune sweep(born::Tune t, int k) {
   return t;
 }
 
-// Autotuner: search tile shape x z chunk for one step kernel and keep the
-// fastest in *tune / *tune_ms (ms per launch).  run(tune) must launch the
-// kernel on scratch buffers only, tiles(shape) is its number of xy tiles (of
-// every shot of a batch), nzi its interior planes (the most of a batch's
-// shots).  xdiv: cells per lane must divide it.
-//
-// z chunks split nzi evenly (ceil(nzi / k) for k chunks, two planes or more):
-// no block marches more planes than the others, and the number of blocks can
-// match what the CUs hold at once.  Which k is best depends on the tile and
-// the grid: a launch wants some hundreds of blocks at least (with 64^3 cells,
-// chunks of 2 planes: 7.4 us per FP32 forward step; of 19 planes, 23.6 us) and
-// few planes read twice (304^3: chunks of 74 planes, 164 us; of 37, 172 us).
-// So each shape (with one plane of lookahead) is first timed with the chunks
-// that come nearest to five numbers of blocks, then the best five shapes with
-// every chunk that gives from half to twice as many blocks as their best, and
-// with two planes of lookahead; the four fastest of all are timed again,
-// round-robin.  The search takes 0.5 s of a 304^3 FP32 pair's first pass,
-// where a grid of every shape and 16 chunk lengths took 1.2 s.
-constexpr int kMinBlocks = 128, kMaxBlocks = 5120;
+// Autotuner: the fastest tile shape and z chunk for one step kernel into *tune
+// and *tune_ms (ms per launch; the search: tune_search.h).  run(tune) must
+// launch the kernel on scratch buffers only, tiles(shape) is its number of xy
+// tiles (of every shot of a batch), nzi its interior planes (the most of a
+// batch's shots).  xdiv: cells per lane must divide it.
 template <class F, class B>
 int autotune_into(born_ctx *ctx, born::Tune *tune, float *tune_ms, int xdiv, int nzi, B tiles,
                   F run) {
@@ -386,10 +373,9 @@ int autotune_into(born_ctx *ctx, born::Tune *tune, float *tune_ms, int xdiv, int
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
-  // ms per launch of `reps` launches, after an untimed one if there are more
-  // than one
-  auto time = [&](const born::Tune &t, int reps, float *ms) -> int {
-    if (reps > 1) HIPCHK(run(sweep(t, 1)));
+  auto time = [&](int shape, int zchunk, int untimed, int reps, float *ms) -> int {
+    const born::Tune t{shape, zchunk};
+    for (int r = 0; r < untimed; r++) HIPCHK(run(sweep(t, 1)));
     HIPCHK(hipEventRecord(e0, ctx->stream));
     for (int r = 0; r < reps; r++) HIPCHK(run(sweep(t, r)));
     HIPCHK(hipEventRecord(e1, ctx->stream));
@@ -398,102 +384,14 @@ int autotune_into(born_ctx *ctx, born::Tune *tune, float *tune_ms, int xdiv, int
     *ms /= reps;
     return BORN_OK;
   };
-  struct Cand {
-    float ms;
-    born::Tune t;
-  };
-  std::vector<Cand> cand;
-  float fastest = 1e30f;
-  auto try_one = [&](int sh, int zc) -> int {
-    for (const Cand &c : cand)
-      if (c.t.shape == sh && c.t.zchunk == zc) return BORN_OK;
-    Cand c{0.f, {sh, zc}};
-    // one launch tells the hopeless ones; launches of a few us are timed over
-    // more of them
-    CHK(time(c.t, 1, &c.ms));
-    if (c.ms < 1.5f * fastest) CHK(time(c.t, c.ms < .03f ? 10 : 3, &c.ms));
-    fastest = std::min(fastest, c.ms);
-    cand.push_back(c);
-    return BORN_OK;
-  };
-  auto faster = [](const Cand &a, const Cand &b) { return a.ms < b.ms; };
-  // the z chunks of a shape with lo to hi blocks, coarse to fine; if none,
-  // the one nearest to that
-  auto chunks = [&](int sh, double lo, double hi) {
-    std::vector<int> zcs;
-    const int n = std::max(1, tiles(sh)), kmax = std::max(1, nzi / 2);
-    int near = 1;
-    for (int k = 1; k <= kmax; k++) {
-      if ((double)n * k < lo) near = k;
-      if ((double)n * k < lo || (double)n * k > hi) continue;
-      const int zc = (nzi + k - 1) / k;
-      if (zcs.empty() || zcs.back() != zc) zcs.push_back(zc);
-    }
-    if (zcs.empty()) zcs.push_back((nzi + near - 1) / near);
-    return zcs;
-  };
-  for (int sh = 0; sh < born::kNumShapes; sh++) {
-    if (xdiv % born::kShapes[sh].vx || born::kShapes[sh].la != 1) continue;
-    if (ctx->zchunk > 0) {
-      CHK(try_one(sh, ctx->zchunk));
-      continue;
-    }
-    const std::vector<int> zcs = chunks(sh, kMinBlocks, kMaxBlocks);
-    const int n = std::max(1, tiles(sh));
-    for (double target : {256., 512., 768., 1280., 2300.}) {
-      int best = zcs[0];
-      double off = 1e30;
-      for (int zc : zcs) {
-        const double nb = (double)n * ((nzi + zc - 1) / zc);
-        const double d = nb > target ? nb / target : target / nb;
-        if (d < off) {
-          off = d;
-          best = zc;
-        }
-      }
-      CHK(try_one(sh, best));
-    }
-  }
-  std::vector<Cand> order = cand;
-  std::sort(order.begin(), order.end(), faster);
-  std::vector<int> done;
-  for (size_t i = 0; i < order.size() && done.size() < 5; i++) {
-    const int sh = order[i].t.shape, zc = order[i].t.zchunk;
-    if (std::find(done.begin(), done.end(), sh) != done.end()) continue;
-    done.push_back(sh);
-    const born::TileShape &ts = born::kShapes[sh];
-    for (int l = 0; l < born::kNumShapes; l++) {
-      const born::TileShape &o = born::kShapes[l];
-      if (o.la == 2 && o.ry == ts.ry && o.wy == ts.wy && o.vx == ts.vx && o.lx == ts.lx)
-        CHK(try_one(l, zc));
-    }
-    if (ctx->zchunk > 0) continue;
-    const double nb = (double)std::max(1, tiles(sh)) * ((nzi + zc - 1) / zc);
-    for (int z : chunks(sh, nb / 2, nb * 2)) CHK(try_one(sh, z));
-  }
-  std::sort(cand.begin(), cand.end(), faster);
-  // the four fastest again, round-robin over three rounds of about 2 ms, 8 to
-  // 30 launches (a drift of the clocks during the search then favours none)
-  const size_t top = std::min<size_t>(cand.size(), 4);
-  const int reps = (int)std::min(30.f, std::max(8.f, 2.f / std::max(cand[0].ms, 1e-3f)));
-  float sum[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int round = 0; round < 3; round++)
-    for (size_t i = 0; i < top; i++) {
-      float ms = 0.f;
-      CHK(time(cand[i].t, reps, &ms));
-      sum[i] += ms / 3.f;
-    }
-  float best = 1e30f;
-  born::Tune bt = *tune;
-  for (size_t i = 0; i < top; i++)
-    if (sum[i] < best) {
-      best = sum[i];
-      bt = cand[i].t;
-    }
+  born::TuneChoice best{tune->shape, tune->zchunk, -1.f};
+  const int rc = born::tune_search(born::kShapes, born::kNumShapes, xdiv, nzi, ctx->zchunk,
+                                   tiles, time, &best);
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  *tune = bt;
-  *tune_ms = best;
+  CHK(rc);
+  *tune = {best.shape, best.zchunk};
+  *tune_ms = best.ms;
   return BORN_OK;
 }
 
