@@ -56,7 +56,7 @@ struct Grid {
   int ntx, nty, ntz;  // tiles along x, y and z chunks
   int zc;             // planes per z chunk
   uint32_t plane;     // nx*ny
-  int back;           // 1: every z chunk is marched the other way
+  int back;           // 1: every z chunk is marched the other way; 2: all are marched up
 };
 
 // Per-axis sponge factors: bound[min(edge_x, edge_y, edge_z)] equals
@@ -745,11 +745,11 @@ __device__ __forceinline__ void march_tile(const Grid &g, const Taps &t, const S
   // The chunk's planes z0 .. z1 - 1.  Chunks are marched up and down in turn,
   // so that two neighbours read the planes they share at about the same time,
   // and a time loop turns every chunk round from one step to the next
-  // (g.back), so that a step starts with the planes the last one ended with.
-  // z is the count of a marched plane, zp its plane in the fields.
+  // (g.back), so that a step starts with the planes the last one ended with
+  // (back 2: all are marched up, see batch_sweep() in born_abi.hip).  z is the count of a marched plane, zp its plane in the fields.
   const int z0 = kH + bz * g.zc;
   const int z1 = min(z0 + g.zc, g.nz - kH);
-  const bool down = ((bz & 1) ^ g.back) != 0;
+  const bool down = g.back < 2 && ((bz & 1) ^ g.back) != 0;
   const int zb = down ? z0 + z1 - 1 : 0, zs = down ? -1 : 1;
   auto zp = [&](int z) { return zb + zs * z; };
   auto zoff = [&](int z) { return (uint32_t)zp(z) * g.plane; };
