@@ -200,6 +200,11 @@ int born_set_step_pairs(born_ctx *ctx, int mode);
 /* bit 0: the last Born forward advanced in two-step launches; bit 1: the
  * last exact adjoint did */
 int born_last_step_pairs(const born_ctx *ctx);
+/* bit 0: the last Born forward held its levels of s and r together, cell by
+ * cell (narrow storage: always; FP32: unless s levels are wanted by
+ * themselves); bit 1: the last reference adjoint did (grids of 2^21 cells and
+ * 48 steps or more).  Results do not depend on it. */
+int born_last_levels_together(const born_ctx *ctx);
 
 /* Placement in HBM of the two levels of the scattered field (Born forward;
  * of s and r together with FP16 or 24-bit storage) and of the adjoint

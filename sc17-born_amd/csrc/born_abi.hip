@@ -123,6 +123,7 @@ struct born_ctx {
   int last_segments = 0, last_recomputed = 0, last_swept = 0;
   int last_pairs = 0;
   int last_lam_pairs = 0;
+  int last_sr = 0;  // bit 0: the last forward held s and r together, bit 1: rtmAdjoint
 
   // Placement of the work pair: the two levels of r of the FP32 forward (of
   // s and r together with narrow storage) and of nu of the adjoint state.
@@ -1320,6 +1321,7 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
   const int fkind = fwd_kind(ctx->storage, scatter);
   const int kind = pair ? sr_kind(fkind) : fkind;
   if (!half) ctx->tuned_sr[fkind] = pair;
+  ctx->last_sr = (ctx->last_sr & ~1) | (half || pair ? 1 : 0);
   // velocity 2 and the model as one stream (8 bytes per cell; the buffer
   // comes with the work buffers)
   HIPCHK(born::launch_interleave(ctx->d_vm, ctx->d_vel2, model, n, ctx->stream));
@@ -1666,6 +1668,7 @@ int born_dev_rtm_adjoint(born_ctx *ctx, int nt, float *p0, float *p1, float *img
   const bool pair = n >= 1 << 21 && nt >= 48;
   const int kind = pair ? K_RADJSR : K_RADJ;
   ctx->tuned_sr[K_RADJ] = pair;
+  ctx->last_sr = (ctx->last_sr & ~2) | (pair ? 2 : 0);
   {  // tune on work fields and the accumulator (no trace read, image untouched)
     born::RadjStep t{};
     t.pair = pair;
@@ -2175,6 +2178,8 @@ int born_set_step_pairs(born_ctx *ctx, int mode) {
 int born_last_step_pairs(const born_ctx *ctx) {
   return ctx ? ctx->last_pairs | ctx->last_lam_pairs << 1 : 0;
 }
+
+int born_last_levels_together(const born_ctx *ctx) { return ctx ? ctx->last_sr : 0; }
 
 int born_set_storage(born_ctx *ctx, int storage) {
   if (!ctx) return BORN_ERR_ARG;

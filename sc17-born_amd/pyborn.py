@@ -62,6 +62,7 @@ SIGNATURES = {
     "born_set_placement": (_i, [_vp, _i, C.c_longlong]),
     "born_last_placement": (_i, [_vp, C.POINTER(_i), C.POINTER(_i)]),
     "born_last_step_pairs": (_i, [_vp]),
+    "born_last_levels_together": (_i, [_vp]),
     "born_set_autotune": (_i, [_vp, _i]),
     "born_get_tuning": (_i, [_vp, _i, C.POINTER(_i), C.POINTER(_i), C.POINTER(_i),
                              C.POINTER(C.c_float)]),
@@ -286,6 +287,13 @@ class Propagator:
     def last_step_pairs(self):
         """True when the last Born forward ran in two-step launches."""
         return bool(self.lib.born_last_step_pairs(self.h) & 1)
+
+    @property
+    def last_levels_together(self):
+        """(Born forward, reference adjoint): s and r together per cell in
+        the levels of the last call."""
+        n = self.lib.born_last_levels_together(self.h)
+        return bool(n & 1), bool(n & 2)
 
     @property
     def last_adjoint_pairs(self):
