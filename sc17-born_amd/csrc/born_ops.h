@@ -262,28 +262,28 @@ struct SrcOp {
   const float *__restrict__ vel;
   Points pts;
   const float *__restrict__ amp;
-  __device__ uint32_t block(int x0, int x1, int y0, int y1, int z0, int z1) const {
-    return points_in_block(pts, x0, x1, y0, y1, z0, z1);
+  __device__ PtsBlk block(int x0, int x1, int y0, int y1, int z0, int z1) const {
+    return points_of_block(pts, x0, x1, y0, y1, z0, z1);
   }
   template <int VX>
-  __device__ void ldv(uint32_t, int, uint32_t po, uint32_t o, float (&v)[VX]) const {
+  __device__ void ldv(const PtsBlk &, int, uint32_t po, uint32_t o, float (&v)[VX]) const {
     ld_vec<VX>(s1, po, o, 1.f, v);
   }
-  __device__ uint32_t plane(uint32_t blk, int z) const {
+  __device__ uint32_t plane(const PtsBlk &blk, int z) const {
     return points_on_plane(pts, blk, z);
   }
   template <int VX>
-  __device__ void prefetchv(uint32_t, float (&p)[NPRE][VX], uint32_t po,
+  __device__ void prefetchv(const PtsBlk &, float (&p)[NPRE][VX], uint32_t po,
                             uint32_t o) const {
     ld_vec<VX>(s0, po, o, 1.f, p[0]);
     ld_vec<VX>(vel, po, o, 1.f, p[1]);
   }
   template <int VX>
-  __device__ void storev(uint32_t, uint32_t po, uint32_t o,
+  __device__ void storev(const PtsBlk &, uint32_t po, uint32_t o,
                          const float (&out)[NOUT][VX]) const {
     st_vec<VX>(s0, po, o, out[0], 1.f);
   }
-  __device__ void cell(uint32_t, uint32_t pm, const CellArgs &c, const float *lap,
+  __device__ void cell(const PtsBlk &, uint32_t pm, const CellArgs &c, const float *lap,
                        const float *ctr, const float *p, float (&out)[NOUT],
                        float (&)[NF]) const {
     float sn = p[1] * lap[0] + ctr[0] + ctr[0] - p[0];
@@ -323,22 +323,22 @@ struct RadjOp {
   __device__ int rec_slot(const SrcPln &pl) const { return gin ? pl.slot : -1; }
   __device__ const int *rec_map(int slot) const { return rec_plane(rm, slot, nx, ny); }
   __device__ float rec_value(int i) const { return gin[i]; }
-  __device__ uint32_t block(int x0, int x1, int y0, int y1, int z0, int z1) const {
-    return pre ? points_in_block(pts, x0, x1, y0, y1, z0, z1) : 0u;
+  __device__ PtsBlk block(int x0, int x1, int y0, int y1, int z0, int z1) const {
+    return pre ? points_of_block(pts, x0, x1, y0, y1, z0, z1) : PtsBlk{0u, 1, 0};
   }
   template <int VX>
-  __device__ void ldv(uint32_t, int f, uint32_t po, uint32_t o, float (&v)[VX]) const {
+  __device__ void ldv(const PtsBlk &, int f, uint32_t po, uint32_t o, float (&v)[VX]) const {
     ld_vec<VX>(f == 0 ? s1 : r1, po, o, 1.f, v);
   }
   template <int VX>
-  __device__ void ldv2(uint32_t, uint32_t po, uint32_t o, float (&v)[2][VX]) const {
+  __device__ void ldv2(const PtsBlk &, uint32_t po, uint32_t o, float (&v)[2][VX]) const {
     ld_vec2<VX>((const float2 *)s1, po, o, v[0], v[1]);
   }
-  __device__ SrcPln plane(uint32_t blk, int z) const {
+  __device__ SrcPln plane(const PtsBlk &blk, int z) const {
     return {points_on_plane(pts, blk, z), ldc(rm.plane_slot, z)};
   }
   template <int VX>
-  __device__ void prefetchv(uint32_t, float (&p)[NPRE][VX], uint32_t po,
+  __device__ void prefetchv(const PtsBlk &, float (&p)[NPRE][VX], uint32_t po,
                             uint32_t o) const {
     if constexpr (PAIRED) {
       ld_vec2<VX>((const float2 *)s0, po, o, p[0], p[1]);
@@ -351,7 +351,7 @@ struct RadjOp {
     ld_vec<VX>(img, po, o, 1.f, p[4]);
   }
   template <int VX>
-  __device__ void storev(uint32_t, uint32_t po, uint32_t o,
+  __device__ void storev(const PtsBlk &, uint32_t po, uint32_t o,
                          const float (&out)[NOUT][VX]) const {
     // no hint: every array here is read again by the next step (304^3 227.9 ->
     // 223.4 us, 160^3 29.4 -> 27.9; with the hint on the loads too, 160^3 35)
@@ -364,7 +364,7 @@ struct RadjOp {
     }
     st_vec<VX, false>(img, po, o, out[2], 1.f);
   }
-  __device__ void cell(uint32_t, const SrcPln &pl, const CellArgs &c, const float *lap,
+  __device__ void cell(const PtsBlk &, const SrcPln &pl, const CellArgs &c, const float *lap,
                        const float *ctr, const float *p, float (&out)[NOUT],
                        float (&)[NF]) const {
     float sn;
