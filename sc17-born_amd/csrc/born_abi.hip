@@ -1318,6 +1318,9 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
   const bool mid = n >= 1 << 19 && n <= (ctx->seg_gap ? 10000000 : 14000000);
   const bool pair = !half && !try_pairs && ckS == 0 &&
                     (!hist || mid || (scatter == 1 && !ctx->seg_gap));
+  // (FwdOp, HINT: levels, velocity and model, 24 bytes per cell; a little later
+  // with the dV term, mostly beside a history)
+  const bool fhint = pair && n * 24 > (scatter == 0 ? 330000000 : 440000000);
   const int fkind = fwd_kind(ctx->storage, scatter);
   const int kind = pair ? sr_kind(fkind) : fkind;
   if (!half) ctx->tuned_sr[fkind] = pair;
@@ -1333,7 +1336,7 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
     t.s1 = ctx->d_w[pair ? 2 : 1]; t.s0 = ctx->d_w[0]; t.r1 = ctx->d_w[3]; t.r0 = ctx->d_w[2];
     t.vel = ctx->d_vel2; t.model = model; t.vm = ctx->d_vm;
     t.src = no_points(); t.rec = recmap(ctx);
-    t.scatter = scatter; t.pair = pair;
+    t.scatter = scatter; t.pair = pair; t.hint = fhint;
     t.h = half_state(ctx, 0);
     t.rg = ctx->d_ring + RING_T0; t.hscale = ctx->d_ring + HS_T;
     // The buffers the steps below use.  With the s levels in the kept
@@ -1392,7 +1395,7 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
     born::FwdStep t{};  // a step without sources or traces
     t.vel = ctx->d_vel2; t.model = model; t.vm = ctx->d_vm; t.src = no_points();
     t.rec = recmap(ctx);
-    t.scatter = scatter;
+    t.scatter = scatter; t.hint = fhint;
     t.h = half_state(ctx, 0); t.rg = ctx->d_ring + RING_T0; t.hscale = ctx->d_ring + HS_T;
     const std::vector<uintptr_t> key = {
         (uintptr_t)ctx->d_seg, ctx->seg_win, (uintptr_t)scatter, (uintptr_t)n,
@@ -1487,6 +1490,7 @@ int born_dev_forward(born_ctx *ctx, int jt, int nt, int scatter, const float *mo
   a.rec = recmap(ctx);
   a.scatter = scatter;
   a.pair = pair;
+  a.hint = fhint;
   a.rg = ctx->d_ring + RING_S;
   // With scatter 0 the scatter operand of step it is s of level it+1, so a
   // kept history holds the s levels: step it reads levels it (history it-1)
@@ -1757,6 +1761,8 @@ int born_dev_adjoint_exact(born_ctx *ctx, int jt, int nt, int scatter,
   const Geometry geo = geometry(ctx);
   const int skind = srec_kind(ctx->storage, scatter);
   const int lkind = lam_kind(ctx->storage);
+  // (SrecOp, HINT: two narrow levels, velocity and image)
+  const bool ahint = half && n * (2 * (long long)esz + 8) > 512000000;
   // bound of |V B P^T w| per unit of max |trace| (FP16 scales)
   const float inj = ctx->vmax2 * ctx->tabd_abs * (float)ctx->rec_per_cell;
   {  // tune both kernels on work fields, the accumulator and scratch scales
@@ -1764,6 +1770,7 @@ int born_dev_adjoint_exact(born_ctx *ctx, int jt, int nt, int scatter,
     HIPCHK(born::launch_fill(ctx->d_ring + MAX_T, 1, 0.f, ctx->stream));
     HIPCHK(born::launch_fill(ctx->d_ring + HS_T, 1, 1.f, ctx->stream));
     born::SrecStep t{};
+    t.hint = ahint;
     t.s1 = ctx->d_w[3]; t.s0 = ctx->d_w[2]; t.vel = ctx->d_vel2; t.sig = ctx->d_acc;
     t.src = no_points(); t.scatter = scatter;
     t.h = half_state(ctx, 0); t.ring = ring(ctx, RING_T0); t.hscale = ctx->d_ring + HS_T;
@@ -1772,6 +1779,7 @@ int born_dev_adjoint_exact(born_ctx *ctx, int jt, int nt, int scatter,
     CHK(ring_reset(ctx, RING_T0));
     HIPCHK(born::launch_fill(ctx->d_ring + HS_T, 1, 1.f, ctx->stream));
     born::LamStep l{};
+    l.hint = ahint;
     l.u1 = ctx->d_w[1]; l.u0 = ctx->d_w[0]; l.vel = ctx->d_vel2; l.sig = ctx->d_w[2];
     l.acc = ctx->d_acc; l.rec = recmap(ctx);
     l.h = half_state(ctx, 0); l.ring = ring(ctx, RING_T0); l.inj = inj;
@@ -1827,6 +1835,7 @@ int born_dev_adjoint_exact(born_ctx *ctx, int jt, int nt, int scatter,
   // that fill the segment history write their s levels straight into it
   const bool s_in_seg = scatter == 0;
   born::SrecStep sr{};
+  sr.hint = ahint;
   sr.vel = ctx->d_vel2;
   sr.src = points(ctx);
   sr.scatter = scatter;
@@ -1879,6 +1888,7 @@ int born_dev_adjoint_exact(born_ctx *ctx, int jt, int nt, int scatter,
   std::vector<int> uplaces;
   if (place) {
     born::LamStep t{};  // a step without receivers
+    t.hint = ahint;
     t.vel = ctx->d_vel2; t.acc = ctx->d_acc; t.rec = recmap(ctx);
     t.h = half_state(ctx, 0); t.ring = ring(ctx, RING_T0); t.inj = inj;
     t.trmax = maxp(ctx, MAX_T); t.hscale = ctx->d_ring + HS_T;
@@ -1913,6 +1923,7 @@ int born_dev_adjoint_exact(born_ctx *ctx, int jt, int nt, int scatter,
                                (unsigned *)(ctx->d_ring + MAX_TR), ctx->stream));
   }
   born::LamStep lm{};
+  lm.hint = ahint;
   lm.vel = ctx->d_vel2;
   float *acc = ctx->d_acc;  // the image accumulator, moved with nu
   lm.rec = recmap(ctx);

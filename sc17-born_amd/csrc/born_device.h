@@ -620,7 +620,7 @@ __device__ __forceinline__ void ld_vec(const __half *p, uint32_t po, uint32_t o,
   }
 }
 // two FP32 fields interleaved cell by cell
-template <int VX>
+template <int VX, bool NT = false>
 __device__ __forceinline__ void ld_vec2(const float2 *p, uint32_t po, uint32_t o,
                                            float (&a)[VX], float (&b)[VX]) {
   const char *q = adv(p, (uint64_t)po * 8u);
@@ -628,7 +628,7 @@ __device__ __forceinline__ void ld_vec2(const float2 *p, uint32_t po, uint32_t o
   for (int h = 0; h < (VX + 1) / 2; h++) {
     constexpr int N = VX == 1 ? 2 : 4;
     uint32_t u[N];
-    ld_words<uint32_t, N>(q + 16 * h, o * 8u, u);
+    ld_words<uint32_t, N, NT>(q + 16 * h, o * 8u, u);
 #pragma unroll
     for (int i = 0; i < N / 2; i++) {
       a[2 * h + i] = __uint_as_float(u[2 * i]);

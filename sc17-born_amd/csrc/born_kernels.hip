@@ -186,6 +186,14 @@ BORN_ALL_TYPES(BORN_FWD_STEP, extern template, 0);
 BORN_ALL_TYPES(BORN_FWD_STEP, extern template, 1);
 BORN_FWD_STEP_SR(extern template, 0);
 BORN_FWD_STEP_SR(extern template, 1);
+BORN_FWD_STEP_HINT(extern template, 0);
+BORN_FWD_STEP_HINT(extern template, 1);
+BORN_SREC_STEP_HINT(extern template, 0, __half);
+BORN_SREC_STEP_HINT(extern template, 1, __half);
+BORN_SREC_STEP_HINT(extern template, 0, Split);
+BORN_SREC_STEP_HINT(extern template, 1, Split);
+BORN_LAM_STEP_HINT(extern template, __half);
+BORN_LAM_STEP_HINT(extern template, Split);
 BORN_ALL_TYPES(BORN_SREC_STEP, extern template, 0);
 BORN_ALL_TYPES(BORN_SREC_STEP, extern template, 1);
 BORN_ALL_TYPES(BORN_LAM_STEP, extern template);
@@ -206,13 +214,18 @@ static hipError_t by_storage(int on, F f) {
 
 hipError_t launch_fwd_step(const Geometry &geo, const Tune &tu, const FwdStep &a,
                            hipStream_t st) {
-  if (a.h.on == 0 && a.pair)
-    return a.scatter == 0 ? fwd_step<0, float, true>(geo, tu, a, st)
-                          : fwd_step<1, float, true>(geo, tu, a, st);
+  const bool s0 = a.scatter == 0;
+  if (a.h.on == 0 && a.pair) {
+    if (a.hint)
+      return s0 ? fwd_step<0, float, true, true>(geo, tu, a, st)
+                : fwd_step<1, float, true, true>(geo, tu, a, st);
+    return s0 ? fwd_step<0, float, true, false>(geo, tu, a, st)
+              : fwd_step<1, float, true, false>(geo, tu, a, st);
+  }
   return by_storage(a.h.on, [&](auto t) {
     using T = decltype(t);
-    return a.scatter == 0 ? fwd_step<0, T, kNarrow<T>>(geo, tu, a, st)
-                          : fwd_step<1, T, kNarrow<T>>(geo, tu, a, st);
+    return s0 ? fwd_step<0, T, kNarrow<T>, false>(geo, tu, a, st)
+              : fwd_step<1, T, kNarrow<T>, false>(geo, tu, a, st);
   });
 }
 
@@ -220,13 +233,23 @@ hipError_t launch_srec_step(const Geometry &geo, const Tune &tu, const SrecStep 
                             hipStream_t st) {
   return by_storage(a.h.on, [&](auto t) {
     using T = decltype(t);
-    return a.scatter == 0 ? srec_step<0, T>(geo, tu, a, st) : srec_step<1, T>(geo, tu, a, st);
+    if constexpr (kNarrow<T>)
+      if (a.hint)
+        return a.scatter == 0 ? srec_step<0, T, true>(geo, tu, a, st)
+                              : srec_step<1, T, true>(geo, tu, a, st);
+    return a.scatter == 0 ? srec_step<0, T, false>(geo, tu, a, st)
+                          : srec_step<1, T, false>(geo, tu, a, st);
   });
 }
 
 hipError_t launch_lam_step(const Geometry &geo, const Tune &tu, const LamStep &a,
                            hipStream_t st) {
-  return by_storage(a.h.on, [&](auto t) { return lam_step<decltype(t)>(geo, tu, a, st); });
+  return by_storage(a.h.on, [&](auto t) {
+    using T = decltype(t);
+    if constexpr (kNarrow<T>)
+      if (a.hint) return lam_step<T, true>(geo, tu, a, st);
+    return lam_step<T, false>(geo, tu, a, st);
+  });
 }
 
 hipError_t launch_batch_fwd_step(const Taps &taps, const Tune &tu, const BatchFwdStep &b,

@@ -67,6 +67,7 @@ struct FwdStep {
   int pair;
   float *rg;  // FP16 ring block: s ring at 0, r ring at 8, max |model| at 16
   float *hscale;
+  bool hint = false;  // the non-temporal hint, for grids past the memory-side cache (born_ops.h)
 };
 
 // Two forward steps in one launch (FP32 levels): reads levels k-1 and k of
@@ -139,6 +140,7 @@ struct SrecStep {
   Half h;
   Ring ring;
   float *hscale;
+  bool hint = false;  // the non-temporal hint, for grids past the memory-side cache (born_ops.h)
 };
 
 struct LamStep {
@@ -153,6 +155,7 @@ struct LamStep {
   float inj;
   const unsigned *trmax;
   const float *hscale;
+  bool hint = false;  // the non-temporal hint, for grids past the memory-side cache (born_ops.h)
 };
 
 // Placement of one shot of a batch inside the batch's arrays (elements).

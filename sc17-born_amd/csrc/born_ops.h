@@ -92,7 +92,19 @@ __device__ __forceinline__ float amp_sum(const Points &pts, const float *amp) {
 // 22.9, 224^3 61.5 -> 51.8, 304^3 173.7 -> 162.9, 203^3 54.6 -> 52.8, 64^3 7.8 ->
 // 7.7; 16 shots of 114-144 x 114-152 x 112 222 -> 188.  FP32 levels stay apart
 // where s levels are wanted by themselves (born_dev_forward).
-template <int SCATTER, class T, bool NT = true, bool PAIR = kNarrow<T>>
+//
+// HINT: FP32 levels together with the non-temporal hint on the old level,
+// velocity and model, and on the stores: for grids whose levels, velocity and
+// model (24 bytes per cell) are past the 256 MB memory-side cache, where what a
+// step leaves there is gone before the next one comes to it, and accesses
+// without the hint only evict the halo rows.  us per step without -> with: 224^3
+// 52 -> 63, 240^3 78.0 -> 78.3, 256^3 92.6 -> 87.4, 304^3 163 -> 146, 384 x 384 x
+// 352 340 -> 306, 448 x 448 x 400 524 -> 469, 640 x 640 x 500 1484 -> 1402 (1394
+// with s and r apart and hints throughout); dV term with its history 240^3 89.4
+// -> 89.0, 256^3 101.9 -> 103.1, 272^3 129.8 -> 126.5, 304^3 187 -> 167.  Narrow
+// levels do without: FP16 gains 1 % from 448^3 on; 24-bit 256^3 80 -> 77, 272 x
+// 288 x 320 (pair) 30.7 -> 31.3 ms, 448 x 448 x 400 445 -> 440.
+template <int SCATTER, class T, bool NT = true, bool PAIR = kNarrow<T>, bool HINT = false>
 struct FwdOp {
   static constexpr bool H = kScaled<T>;
   static constexpr int NF = 2, NPRE = 4, NOUT = 3, NMAX = H ? 2 : 0, REC = 1;
@@ -102,7 +114,7 @@ struct FwdOp {
   static constexpr bool Q2 = kNarrow<T>;  // steps in pairs (march_tile)
   // (FP32, s and r together: 22.8 us per step without, 23.4 with, at 160^3,
   // where the registers are not what limits the wavefronts)
-  static constexpr bool LEAN = kNarrow<T> || !PAIR;
+  static constexpr bool LEAN = kNarrow<T> || !PAIR || HINT;
   static constexpr bool DAMP = true;
   const T *__restrict__ s1;
   const T *__restrict__ r1;
@@ -191,7 +203,10 @@ struct FwdOp {
                             uint32_t o) const {
     if constexpr (PAIRED) {
       float sr[2][VX];
-      ld_pair<VX>(sr0, po, o, b.io, sr, nlev);
+      if constexpr (HINT)
+        ld_vec2<VX, true>(sr0, po, o, sr[0], sr[1]);
+      else
+        ld_pair<VX>(sr0, po, o, b.io, sr, nlev);
 #pragma unroll
       for (int v = 0; v < VX; v++) {
         p[0][v] = sr[0][v];
@@ -205,7 +220,7 @@ struct FwdOp {
       ld_vec<VX>(r0, po, o, b.io[1], p[1], nlev);
     }
     if constexpr (NT) {
-      ld_vec2<VX>(vm, po, o, p[2], p[3]);
+      ld_vec2<VX, HINT>(vm, po, o, p[2], p[3]);
     } else {
       ld_vec<VX>(vel, po, o, 1.f, p[2]);
       ld_vec<VX>(model, po, o, 1.f, p[3]);
@@ -215,7 +230,7 @@ struct FwdOp {
   __device__ void storev(const Blk2 &b, uint32_t po, uint32_t o,
                          const float (&out)[NOUT][VX]) const {
     if constexpr (PAIRED) {
-      st_pair<VX, false>(srn, po, o, out[0], out[1], b.sn, nlev);
+      st_pair<VX, HINT>(srn, po, o, out[0], out[1], b.sn, nlev);
     } else {
       st_vec<VX, NT>(s_new, po, o, out[0], b.sn[0], nlev);
       st_vec<VX, NT>(r0, po, o, out[1], b.sn[1], nlev);
@@ -390,7 +405,13 @@ struct RadjOp {
 };
 
 // ------------------------------------- exact adjoint: background recompute
-template <int SCATTER, class T>
+// HINT: narrow levels with the non-temporal hint on the stores and the
+// velocity, for grids past the memory-side cache; the same bit of LamOp, where
+// the image takes it too.  us per step of both without -> with: FP16 304^3 172 ->
+// 185, 384 x 384 x 352 308 -> 291, 448 x 448 x 400 489 -> 463, 640 x 640 x 500 1464
+// -> 1350; 24-bit 304^3 233 -> 244, 384 x 384 x 352 409 -> 409, 448 x 448 x 400 674
+// -> 642, 640 x 640 x 500 1875 -> 1744.
+template <int SCATTER, class T, bool HINT = false>
 struct SrecOp {
   static constexpr bool H = kScaled<T>;
   static constexpr int NF = 1, NPRE = 2, NOUT = 2, NMAX = H ? 1 : 0, REC = 0;
@@ -447,16 +468,16 @@ struct SrecOp {
   __device__ void prefetchv(const Blk1 &b, float (&p)[NPRE][VX], uint32_t po,
                             uint32_t o) const {
     // FP32: the old level and the stores with the non-temporal hint; narrow
-    // levels without any (FP16 background and adjoint state, us per step of
+    // levels without any, but see HINT (FP16 background and adjoint state, us per step of
     // each together: 304^3 196.9 -> 184.9, 160^3 49.7 -> 47.1)
     ld_vec<VX, !kNarrow<T>>(s0, po, o, b.io, p[0], nlev);
-    ld_vec<VX>(vel, po, o, 1.f, p[1]);
+    ld_vec<VX, HINT>(vel, po, o, 1.f, p[1]);
   }
   template <int VX>
   __device__ void storev(const Blk1 &b, uint32_t po, uint32_t o,
                          const float (&out)[NOUT][VX]) const {
-    st_vec<VX, !kNarrow<T>>(s_new, po, o, out[0], b.sn, nlev);
-    if (sig) st_vec<VX, !kNarrow<T>>(sig, po, o, out[1], b.sh, nlev);
+    st_vec<VX, !kNarrow<T> || HINT>(s_new, po, o, out[0], b.sn, nlev);
+    if (sig) st_vec<VX, !kNarrow<T> || HINT>(sig, po, o, out[1], b.sh, nlev);
   }
   __device__ void cell(const Blk1 &, uint32_t pm, const CellArgs &c, const float *lap,
                        const float *ctr, const float *p, float (&out)[NOUT],
@@ -473,7 +494,7 @@ struct SrecOp {
 // ---------------------------------------- exact adjoint: adjoint-state step
 // nu = V B lambda obeys the forward recursion with V B-weighted receiver
 // injection; the image accumulates sigma * nu and is divided by V B at the end.
-template <class T>
+template <class T, bool HINT = false>
 struct LamOp {
   static constexpr bool H = kScaled<T>;
   static constexpr int NF = 1, NPRE = 4, NOUT = 2, NMAX = H ? 1 : 0, REC = 2;
@@ -530,18 +551,18 @@ struct LamOp {
   __device__ void prefetchv(const Blk1 &b, float (&p)[NPRE][VX], uint32_t po,
                             uint32_t o) const {
     // FP32: the non-temporal hint on the levels, not on velocity and image
-    // (304^3 134.8 us; without any 143.5); narrow levels without any (24-bit
-    // 224^3 61.7 -> 58.4)
+    // (304^3 134.8 us; without any 143.5); narrow levels without any, but see
+    // HINT at SrecOp (24-bit 224^3 61.7 -> 58.4)
     ld_vec<VX, !kNarrow<T>>(u0, po, o, b.io, p[0], nlev);
     ld_vec<VX, !kNarrow<T>>(sig, po, o, b.sh, p[2], nlev);
-    ld_vec<VX>(vel, po, o, 1.f, p[1]);
-    ld_vec<VX>(acc, po, o, 1.f, p[3]);
+    ld_vec<VX, HINT>(vel, po, o, 1.f, p[1]);
+    ld_vec<VX, HINT>(acc, po, o, 1.f, p[3]);
   }
   template <int VX>
   __device__ void storev(const Blk1 &b, uint32_t po, uint32_t o,
                          const float (&out)[NOUT][VX]) const {
-    st_vec<VX, !kNarrow<T>>(u0, po, o, out[0], b.sn, nlev);
-    st_vec<VX, false>(acc, po, o, out[1], 1.f);
+    st_vec<VX, !kNarrow<T> || HINT>(u0, po, o, out[0], b.sn, nlev);
+    st_vec<VX, HINT>(acc, po, o, out[1], 1.f);
   }
   __device__ void cell(const Blk1 &, int slot, const CellArgs &c, const float *lap,
                        const float *ctr, const float *p, float (&out)[NOUT],
@@ -804,9 +825,9 @@ hipError_t launch_batch(const Taps &taps, const Tune &tu, const BatchCommon &b,
 // instantiated explicitly, each in one translation unit (born_k_*.hip, built
 // in parallel); born_kernels.hip declares them extern and dispatches.
 
-template <int SCATTER, class T, bool PAIR>
+template <int SCATTER, class T, bool PAIR, bool HINT>
 hipError_t fwd_step(const Geometry &geo, const Tune &tu, const FwdStep &a, hipStream_t st) {
-  FwdOp<SCATTER, T, true, PAIR> op{};
+  FwdOp<SCATTER, T, true, PAIR, HINT> op{};
   op.s1 = as<T>(a.s1); op.r1 = as<T>(a.r1); op.s0 = as<T>(a.s0); op.r0 = as<T>(a.r0);
   op.s_new = as<T>(a.s_new ? a.s_new : a.s0);
   op.sr1 = (const PairOf<T> *)a.s1; op.sr0 = (const PairOf<T> *)a.s0;
@@ -832,9 +853,9 @@ hipError_t radj_step(const Geometry &geo, const Tune &tu, const RadjStep &a, hip
   return launch(geo, tu, op, st);
 }
 
-template <int SCATTER, class T>
+template <int SCATTER, class T, bool HINT>
 hipError_t srec_step(const Geometry &geo, const Tune &tu, const SrecStep &a, hipStream_t st) {
-  SrecOp<SCATTER, T> op{};
+  SrecOp<SCATTER, T, HINT> op{};
   op.s1 = as<T>(a.s1); op.s0 = as<T>(a.s0); op.vel = a.vel; op.sig = as<T>(a.sig);
   op.s_new = as<T>(a.s_new ? a.s_new : a.s0);
   op.pts = to_points(a.src); op.amp = a.amp;
@@ -844,9 +865,9 @@ hipError_t srec_step(const Geometry &geo, const Tune &tu, const SrecStep &a, hip
   return launch(geo, tu, op, st);
 }
 
-template <class T>
+template <class T, bool HINT>
 hipError_t lam_step(const Geometry &geo, const Tune &tu, const LamStep &a, hipStream_t st) {
-  LamOp<T> op{};
+  LamOp<T, HINT> op{};
   op.u1 = as<T>(a.u1); op.u0 = as<T>(a.u0); op.vel = a.vel; op.sig = as<T>(a.sig);
   op.acc = a.acc; op.rm = a.rec; op.gin = a.gin; op.nx = geo.nx; op.ny = geo.ny;
   op.ring = a.ring; op.sl = a.h.sl; op.gain = a.h.gain; op.inj = a.inj;
@@ -904,17 +925,27 @@ hipError_t batch_lam_step(const Taps &taps, const Tune &tu, const BatchLamStep &
 
 // the instantiations, one translation unit each (F: template or extern template)
 #define BORN_FWD_STEP(F, S, T)                                                          \
-  F hipError_t fwd_step<S, T, kNarrow<T>>(const Geometry &, const Tune &, const FwdStep &, \
-                                          hipStream_t)
+  F hipError_t fwd_step<S, T, kNarrow<T>, false>(const Geometry &, const Tune &,         \
+                                                 const FwdStep &, hipStream_t)
 // FP32 levels of s and r together
 #define BORN_FWD_STEP_SR(F, S) \
-  F hipError_t fwd_step<S, float, true>(const Geometry &, const Tune &, const FwdStep &, hipStream_t)
+  F hipError_t fwd_step<S, float, true, false>(const Geometry &, const Tune &,           \
+                                               const FwdStep &, hipStream_t)
+// the same with the non-temporal hint
+#define BORN_FWD_STEP_HINT(F, S)                                                        \
+  F hipError_t fwd_step<S, float, true, true>(const Geometry &, const Tune &,            \
+                                              const FwdStep &, hipStream_t)
 #define BORN_RADJ_STEP(F, PAIR) \
   F hipError_t radj_step<PAIR>(const Geometry &, const Tune &, const RadjStep &, hipStream_t)
 #define BORN_SREC_STEP(F, S, T) \
-  F hipError_t srec_step<S, T>(const Geometry &, const Tune &, const SrecStep &, hipStream_t)
+  F hipError_t srec_step<S, T, false>(const Geometry &, const Tune &, const SrecStep &, hipStream_t)
+// narrow levels with the hint
+#define BORN_SREC_STEP_HINT(F, S, T) \
+  F hipError_t srec_step<S, T, true>(const Geometry &, const Tune &, const SrecStep &, hipStream_t)
 #define BORN_LAM_STEP(F, T) \
-  F hipError_t lam_step<T>(const Geometry &, const Tune &, const LamStep &, hipStream_t)
+  F hipError_t lam_step<T, false>(const Geometry &, const Tune &, const LamStep &, hipStream_t)
+#define BORN_LAM_STEP_HINT(F, T) \
+  F hipError_t lam_step<T, true>(const Geometry &, const Tune &, const LamStep &, hipStream_t)
 #define BORN_BATCH_SREC_STEP(F, S, T)                                                   \
   F hipError_t batch_srec_step<S, T>(const Taps &, const Tune &, const BatchSrecStep &, \
                                      hipStream_t)

@@ -67,10 +67,10 @@ def kernels():
 # two rows per lane, one cell per lane: the shapes whose rows and fields were
 # held in registers together (128 registers: four wavefronts a SIMD)
 @pytest.mark.parametrize("op,shape", [
-    ("FwdOp<0, float, true, false>", "2, 4, 1, 1, 64"),
-    ("FwdOp<0, float, true, false>", "2, 8, 1, 1, 64"),
-    ("FwdOp<0, __half, true, true>", "2, 4, 1, 1, 64"),
-    ("FwdOp<0, __half, true, true>", "2, 8, 1, 2, 64")])
+    ("FwdOp<0, float, true, false, false>", "2, 4, 1, 1, 64"),
+    ("FwdOp<0, float, true, false, false>", "2, 8, 1, 1, 64"),
+    ("FwdOp<0, __half, true, true, false>", "2, 4, 1, 1, 64"),
+    ("FwdOp<0, __half, true, true, false>", "2, 8, 1, 2, 64")])
 def test_four_wavefronts_per_simd(kernels, op, shape):
     k = kernels["march_kernel<%s, %s>" % (op, shape)]
     assert k[".private_segment_fixed_size"] == 0
