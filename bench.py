@@ -57,7 +57,9 @@ METRIC = "Born fwd+adj Mcell-updates/s + HBM GB/s vs peak; FP16-store batch vs F
 # rocprofv3 FETCH_SIZE (x2.0) and WRITE_SIZE (x1.0) runs of this script
 # (profiles/born_fwd_adj_304cube_hbm_counters.md); reported as roofline.traffic
 # only when the measured workload, kernel and z chunk are the profiled ones.
-PROFILED_TRAFFIC = {("c2", "FwdOp<0, float, true>, 2, 4, 1, 1, 64", 74, "f32"): 961.7e6}
+PROFILED_TRAFFIC = {("c2", "FwdOp<0, float, true>, 1, 2, 4, 1, 16", 74, "f32"): 933.0e6,
+                    ("c2", "FwdOp<0, float, true>, 2, 4, 1, 1, 64", 74, "f32"): 951.2e6,
+                    ("c2", "FwdOp<0, float, true>, 1, 4, 4, 1, 16", 60, "f32"): 970.1e6}
 
 
 def load(name):

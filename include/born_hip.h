@@ -232,9 +232,9 @@ int born_last_placement(const born_ctx *ctx, int *forward_moves, int *adjoint_mo
 int born_set_zchunk(born_ctx *ctx, int zchunk);
 
 /* Autotuner of the step kernels' launch shape (on by default): before the
- * first launch of a step kernel on a new grid, every tile shape (rows per
- * thread x wavefronts per block) and z chunk is timed on scratch fields and
- * the fastest kept.  on = 0 keeps the default shape; on = 1 re-tunes. */
+ * first launch of a step kernel on a new grid, tile shapes (rows per thread x
+ * wavefronts per block x cells per lane) and z chunks are timed on scratch
+ * fields, coarse to fine, and the fastest kept.  on = 0 keeps the default shape; on = 1 re-tunes. */
 int born_set_autotune(born_ctx *ctx, int on);
 /* The chosen launch shape of a step kernel: 0 Born forward, 1 Born forward
  * (dV scatter), 2 source propagation, 3 reference adjoint, 4/5 background
@@ -246,8 +246,8 @@ int born_get_tuning(const born_ctx *ctx, int kernel, int *rows_per_thread,
                     int *waves_per_block, int *zchunk, float *ms);
 
 /* The chosen tile of a step kernel: tile_x x tile_y cells of the xy plane,
- * cells_per_lane consecutive x cells per thread (2: one 8-byte / 4-byte load
- * of a pair; needs an even nx), lookahead = how many z planes ahead of the
+ * cells_per_lane consecutive x cells per thread (1, 2 or 4, of which nx is a
+ * multiple: one load for all of them), lookahead = how many z planes ahead of the
  * plane being computed the loads are issued (1 or 2; 1 for the two-step
  * kernels). */
 int born_get_tile(const born_ctx *ctx, int kernel, int *tile_x, int *tile_y,

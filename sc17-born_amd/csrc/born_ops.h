@@ -76,15 +76,16 @@ __device__ __forceinline__ float amp_sum(const Points &pts, const float *amp) {
 }
 
 // ---------------------------------------------------------------- forward
-// NT: the single-shot forward: non-temporal hint on the FP32 and 24-bit
-// stores, velocity and model as one stream (the shot batch: see BatchFwd).
-// The loads take no hint (but see s0): what a step reads the next one reads or overwrites,
-// and a load with the hint leaves nothing in the 256 MB memory-side cache.
-// FP32, us per step with the hint on the pointwise loads -> without: 160^3
-// 31.6 -> 26.4 (dV scatter 35.5 -> 26.1), 224^3 73.7 -> 63.9 (83.7 -> 61.7),
-// 304^3 175.1 -> 172.6 (207.6 -> 194.1).  The stores keep it in FP32: 304^3
-// 172.4 with, 177.9 without.  FP16 without any: 160^3 38.1 -> 36.1, 224^3 72.8
-// -> 66.9, 304^3 127.9 -> 128.9.
+// NT: the single-shot forward: velocity and model as one stream, the
+// non-temporal hint on the stores of levels apart and of the history (the shot
+// batch: see BatchFwd).  The other accesses take no hint (but see s0 and HINT):
+// what a step reads the next one reads or overwrites, and an access with the
+// hint leaves nothing in the 256 MB memory-side cache.  FP32, us per step with
+// the hint on the pointwise loads -> without: 160^3 31.6 -> 26.4 (dV scatter 35.5
+// -> 26.1), 224^3 73.7 -> 63.9 (83.7 -> 61.7).  Levels apart are those of large
+// grids: 304^3 172.4 with the hint on their stores, 177.9 without.  No step reads
+// the history again.  FP16 levels with the hint -> without: 160^3 38.1 -> 36.1,
+// 224^3 72.8 -> 66.9, 304^3 127.9 -> 128.9.
 //
 // PAIR: s and r together per cell.  Half as many streams, twice as long: rows
 // of a level are seldom whole cache lines, and each tile's row ends in two
@@ -127,7 +128,7 @@ struct FwdOp {
   const PairOf<T> *sr1;
   const PairOf<T> *sr0;
   PairOf<T> *srn;
-  const float *__restrict__ vel;
+  const float *__restrict__ vel;  // vel and model: the shot batch
   const float *__restrict__ model;
   // NT (the single-shot forward): vel and model interleaved per cell, one
   // load and one stream for both
@@ -603,11 +604,6 @@ struct BatchFwd {
     r.sp.bz = sponge + d.sp0 + d.nx + d.ny;
     Op &o = r.op;
     o = base;
-    o.s1 = base.s1 + d.cell0;
-    o.r1 = base.r1 + d.cell0;
-    o.s0 = base.s0 + d.cell0;
-    o.s_new = base.s_new + d.cell0;
-    o.r0 = base.r0 + d.cell0;
     o.sr1 = base.sr1 + d.cell0;
     o.sr0 = base.sr0 + d.cell0;
     o.srn = base.srn + d.cell0;
@@ -720,7 +716,6 @@ struct BatchLam {
 // ------------------------------------------------------------- launchers
 
 // switch (shape) { case i: return F<..., RY, WY, VX, LA, LX>(ARGS); } over kShapes
-// switch (shape) { case i: return F<..., RY, WY, VX, LA, LX>(ARGS); } over kShapes
 #define BORN_SHAPE_CASES(F, OP, ...)                         \
   case 0: return F<OP, 2, 4, 1, 1, 64>(__VA_ARGS__);         \
   case 1: return F<OP, 4, 4, 1, 1, 64>(__VA_ARGS__);         \
@@ -832,7 +827,7 @@ hipError_t fwd_step(const Geometry &geo, const Tune &tu, const FwdStep &a, hipSt
   op.s_new = as<T>(a.s_new ? a.s_new : a.s0);
   op.sr1 = (const PairOf<T> *)a.s1; op.sr0 = (const PairOf<T> *)a.s0;
   op.srn = (PairOf<T> *)(a.s_new ? a.s_new : a.s0);
-  op.vel = a.vel; op.model = a.model; op.vm = (const float2 *)a.vm; op.hist = as<T>(a.hist);
+  op.vm = (const float2 *)a.vm; op.hist = as<T>(a.hist);
   if (!a.vm) return hipErrorInvalidValue;
   op.pts = to_points(a.src); op.amp = a.amp;
   op.rm = a.rec; op.rv = a.rv; op.nx = geo.nx; op.ny = geo.ny;
@@ -882,8 +877,6 @@ hipError_t batch_fwd_step(const Taps &taps, const Tune &tu, const BatchFwdStep &
   const FwdStep &a = b.a;
   BatchFwd<SCATTER, T> bop{};
   auto &op = bop.base;
-  op.s1 = as<T>(a.s1); op.r1 = as<T>(a.r1); op.s0 = as<T>(a.s0); op.r0 = as<T>(a.r0);
-  op.s_new = as<T>(a.s0);
   op.sr1 = (const PairOf<T> *)a.s1; op.sr0 = (const PairOf<T> *)a.s0;
   op.srn = (PairOf<T> *)a.s0;
   op.vel = a.vel; op.model = a.model; op.hist = nullptr;
